@@ -164,11 +164,11 @@ __global__ void __launch_bounds__(256) ce_head_rows(CeHeadParams p) {
     for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
   };
-  const float e2 = cls ? (float)exp((double)(z - m2)) : 0.0f;
+  const float e2 = cls ? exp_rn(z - m2) : 0.0f;
   const double s2 = sum16(cls ? (double)e2 : 0.0);
   const float sum2 = (float)s2;
   double s = s2;
-  if (!(m == m2)) s = sum16(cls ? (double)(float)exp((double)(z - m)) : 0.0);  // a NaN logit
+  if (!(m == m2)) s = sum16(cls ? (double)exp_rn(z - m) : 0.0);  // a NaN logit
   const float lse = m + (float)log((double)(float)s);
   if (lane == 0) p.row_loss[r] = in_range ? lse - zt : 0.0f;
   const int64_t safe = t < 0 ? 0 : (t >= J ? J - 1 : t);

@@ -11,6 +11,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "fexp64.h"
 #include "kernels.h"
 
 namespace shk {
@@ -33,20 +34,9 @@ __device__ __forceinline__ float relu_f(float x) {
   return (x > 0.0f || x != x) ? x : 0.0f;
 }
 
-// Stable two-branch logistic in binary64 (CpuScalarReferenceKernel.java:1213-1217).
-__device__ __forceinline__ float sigmoid_f(float xf) {
-  double x = (double)xf;
-  double r;
-  if (x >= 0.0) {
-    r = 1.0 / (1.0 + exp(-x));
-  } else {
-    double e = exp(x);
-    r = e / (1.0 + e);
-  }
-  return (float)r;
-}
-
-__device__ __forceinline__ float tanh_f(float x) { return (float)tanh((double)x); }
+// Binary64 evaluations rounded once (fexp64.h).
+__device__ __forceinline__ float sigmoid_f(float x) { return sigmoid_rn(x); }
+__device__ __forceinline__ float tanh_f(float x) { return tanh_rn(x); }
 
 __device__ __forceinline__ float apply_act(int act, float z) {
   switch (act) {

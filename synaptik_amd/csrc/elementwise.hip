@@ -42,7 +42,7 @@ constexpr int PW_REGS = 8;
 // them into every interpreter case inflates the register allocation of the whole kernel.
 __device__ __noinline__ float pw_tanh(float a) { return tanh_f(a); }
 __device__ __noinline__ float pw_sigmoid(float a) { return sigmoid_f(a); }
-__device__ __noinline__ float pw_exp(float a) { return (float)exp((double)a); }
+__device__ __noinline__ float pw_exp(float a) { return exp_rn(a); }
 __device__ __noinline__ float pw_log(float a) { return (float)log((double)a); }
 __device__ __noinline__ float pw_sqrt(float a) { return (float)sqrt((double)a); }
 
@@ -362,7 +362,7 @@ __global__ void __launch_bounds__(NT) row_reduce_kernel(const float* __restrict_
     // LOG_SUM_EXP: shifted exponentials, one logarithm (CpuLogSumExpEmitter.java:4-9).
     const float shift = (m == INFINITY || m == -INFINITY) ? 0.0f : m;
     double s = 0.0;
-    for (int64_t c = threadIdx.x; c < C; c += NT) s += (double)(float)exp((double)(row[c] - shift));
+    for (int64_t c = threadIdx.x; c < C; c += NT) s += (double)exp_rn(row[c] - shift);
     s = block_sum<NT>(s, dl);
     if (threadIdx.x == 0) {
       float r;

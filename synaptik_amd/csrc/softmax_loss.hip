@@ -349,7 +349,7 @@ __global__ void lse_bwd_kernel(const float* __restrict__ x, const float* __restr
        i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t r = i / C;
     const float gr = g != nullptr ? g[r] : gconst;
-    dx[i] = gr * (float)exp((double)(x[i] - lse[r]));
+    dx[i] = gr * exp_rn(x[i] - lse[r]);
   }
 }
 
@@ -445,7 +445,7 @@ __global__ void __launch_bounds__(256) ce_pass1(const float* __restrict__ logits
           if (u > m) m = u;
         }
         double s = 0.0;
-        for (int64_t c = lane; c < C; c += 64) s += (double)(float)exp((double)(row[c] - m));
+        for (int64_t c = lane; c < C; c += 64) s += (double)exp_rn(row[c] - m);
         s = wave_sum(s);
         const float lse = m + (float)log((double)(float)s);
         loss = (double)(lse - row[t]);
@@ -517,10 +517,10 @@ __global__ void __launch_bounds__(256) ce_grad(const float* __restrict__ logits,
   for (int64_t c = lane; c < C; c += 64) m = java_max(m, row[c]);
   m = wave_max(m);
   double s = 0.0;
-  for (int64_t c = lane; c < C; c += 64) s += (double)(float)exp((double)(row[c] - m));
+  for (int64_t c = lane; c < C; c += 64) s += (double)exp_rn(row[c] - m);
   const float sum = (float)wave_sum(s);
   for (int64_t c = lane; c < C; c += 64) {
-    const float prob = (float)exp((double)(row[c] - m)) / sum;
+    const float prob = exp_rn(row[c] - m) / sum;
     const float hot = c == safe ? 1.0f : 0.0f;
     gr[c] = (prob - hot) * scale;
   }
