@@ -1,4 +1,4 @@
-// Row softmax / log-softmax / log-sum-exp and the MSE and index categorical cross-entropy losses.
+// Row softmax / log-softmax / log-sum-exp and the MSE loss.
 //
 // Softmax follows CpuSoftmaxReferenceKernel.evaluateFloat (reference/CpuSoftmaxReferenceKernel.java:104-146):
 //   maximum by Math.max; a +inf maximum maps +inf entries to NaN and the rest to 0 (softmax) or
@@ -413,119 +413,6 @@ __global__ void __launch_bounds__(256) mse_pass2(const double* part, int P, int6
   if (threadIdx.x == 0) loss[0] = mse_loss(s, n, reduction_sum);
 }
 
-// ---- Index categorical cross-entropy (CpuLossReferenceKernel.java:196-218,261-288;
-//      LossGradientRules.java:172-240). One wave per sample row. ----
-template <typename T>
-__global__ void __launch_bounds__(256) ce_pass1(const float* __restrict__ logits,
-                                                const T* __restrict__ target, int64_t R,
-                                                int64_t C, int has_ignore, int64_t ignore,
-                                                double* part, uint32_t* status) {
-  __shared__ double dl[4];
-  __shared__ double dc[4];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t r = (int64_t)blockIdx.x * 4 + w;
-  double loss = 0.0, count = 0.0;
-  if (r < R) {
-    const int64_t t = (int64_t)target[r];
-    const bool ignored = has_ignore && t == ignore;
-    if (!ignored) {
-      if (t < 0 || t >= C) {
-        if (lane == 0) atomicOr(status, (uint32_t)DEV_INDEX_OUT_OF_BOUNDS);
-      } else {
-        const float* row = logits + r * C;
-        // maximum by '>' (a NaN logit never becomes the maximum), as the loss oracle does
-        float m = -INFINITY;
-        for (int64_t c = lane; c < C; c += 64) {
-          const float v = row[c];
-          if (v > m) m = v;
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-          const float u = __shfl_xor(m, o, 64);
-          if (u > m) m = u;
-        }
-        double s = 0.0;
-        for (int64_t c = lane; c < C; c += 64) s += (double)exp_rn(row[c] - m);
-        s = wave_sum(s);
-        const float lse = m + (float)log((double)(float)s);
-        loss = (double)(lse - row[t]);
-        count = 1.0;
-      }
-    }
-  }
-  if (lane != 0) { loss = 0.0; count = 0.0; }
-  if (lane == 0) { dl[w] = loss; dc[w] = count; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = ((dl[0] + dl[1]) + dl[2]) + dl[3];
-    part[2 * blockIdx.x + 1] = ((dc[0] + dc[1]) + dc[2]) + dc[3];
-  }
-}
-__device__ __forceinline__ void ce_finish(double* part, int P, float* loss, double* dl) {
-  double s = 0.0, c = 0.0;
-  for (int i = threadIdx.x; i < P; i += 256) {
-    s += part[2 * i];
-    c += part[2 * i + 1];
-  }
-  s = block_sum<256>(s, dl);
-  __syncthreads();
-  c = block_sum<256>(c, dl);
-  if (threadIdx.x == 0) {
-    loss[0] = (float)s / (float)c;
-    part[2 * P] = c;  // non-ignored sample count for the gradient pass
-  }
-}
-__global__ void __launch_bounds__(256) ce_pass2(double* part, int P, float* loss) {
-  __shared__ double dl[4];
-  ce_finish(part, P, loss, dl);
-}
-// Gradient rows. FUSED: the launch is the one after ce_pass1 (no ce_pass2): block 0 first does
-// ce_pass2's work (same code, same order), and every block sums the P exact per-block sample
-// counts itself (integers in binary64, exact in any order) instead of reading the total.
-template <typename T, bool FUSED>
-__global__ void __launch_bounds__(256) ce_grad(const float* __restrict__ logits,
-                                               const T* __restrict__ target, int64_t R, int64_t C,
-                                               int has_ignore, int64_t ignore, float g,
-                                               double* part, int P, float* loss,
-                                               float* __restrict__ grad) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  double count;
-  if (FUSED) {
-    __shared__ double dl[4];
-    if (blockIdx.x == 0) {
-      ce_finish(part, P, loss, dl);
-      __syncthreads();
-    }
-    double c = 0.0;
-    for (int i = threadIdx.x; i < P; i += 256) c += part[2 * i + 1];
-    count = block_sum<256>(c, dl);
-  } else {
-    count = part[2 * P];
-  }
-  const int64_t r = (int64_t)blockIdx.x * 4 + w;
-  if (r >= R) return;
-  const int64_t t = (int64_t)target[r];
-  const float* row = logits + r * C;
-  float* gr = grad + r * C;
-  if (has_ignore && t == ignore) {
-    for (int64_t c = lane; c < C; c += 64) gr[c] = 0.0f;
-    return;
-  }
-  const float scale = g / (float)count;
-  const int64_t safe = t < 0 ? 0 : (t >= C ? C - 1 : t);
-  float m = -INFINITY;
-  for (int64_t c = lane; c < C; c += 64) m = java_max(m, row[c]);
-  m = wave_max(m);
-  double s = 0.0;
-  for (int64_t c = lane; c < C; c += 64) s += (double)exp_rn(row[c] - m);
-  const float sum = (float)wave_sum(s);
-  for (int64_t c = lane; c < C; c += 64) {
-    const float prob = exp_rn(row[c] - m) / sum;
-    const float hot = c == safe ? 1.0f : 0.0f;
-    gr[c] = (prob - hot) * scale;
-  }
-}
-
 }  // namespace
 
 hipError_t launch_softmax_fwd(const float* x, float* y, float* lse, int64_t R, int64_t C,
@@ -582,49 +469,6 @@ hipError_t launch_mse(const float* p, const float* t, float* loss, float* grad, 
   if (blocks > 1)
     hipLaunchKernelGGL(mse_pass2, dim3(1), dim3(256), 0, s, (const double*)partial, (int)blocks,
                        n, reduction_sum, loss);
-  return hipGetLastError();
-}
-
-constexpr unsigned CE_FUSE_BLOCKS = 1024;
-int64_t index_ce_partial_doubles(int64_t R) { return 2 * ((R + 3) / 4) + 2; }
-hipError_t launch_index_ce(const float* logits, const void* target, int target_is_64,
-                           float* loss, float* grad, int64_t R, int64_t C, int has_ignore,
-                           int64_t ignore_index, float g, double* partial, uint32_t* status,
-                           hipStream_t s) {
-  if (R <= 0) return hipSuccess;
-  const unsigned blocks = (unsigned)((R + 3) / 4);
-  if (target_is_64)
-    hipLaunchKernelGGL(ce_pass1<int64_t>, dim3(blocks), dim3(256), 0, s, logits,
-                       (const int64_t*)target, R, C, has_ignore, ignore_index, partial, status);
-  else
-    hipLaunchKernelGGL(ce_pass1<int32_t>, dim3(blocks), dim3(256), 0, s, logits,
-                       (const int32_t*)target, R, C, has_ignore, ignore_index, partial, status);
-  const int P = (int)blocks;
-  // Up to CE_FUSE_BLOCKS blocks, the gradient launch also finishes the loss (each block re-sums
-  // the P counts: 2P doubles read per block); beyond that a separate one-block pass does.
-  const bool fuse = grad != nullptr && blocks <= CE_FUSE_BLOCKS;
-  if (!fuse) hipLaunchKernelGGL(ce_pass2, dim3(1), dim3(256), 0, s, partial, P, loss);
-  if (grad != nullptr) {
-    if (target_is_64) {
-      if (fuse)
-        hipLaunchKernelGGL((ce_grad<int64_t, true>), dim3(blocks), dim3(256), 0, s, logits,
-                           (const int64_t*)target, R, C, has_ignore, ignore_index, g, partial, P,
-                           loss, grad);
-      else
-        hipLaunchKernelGGL((ce_grad<int64_t, false>), dim3(blocks), dim3(256), 0, s, logits,
-                           (const int64_t*)target, R, C, has_ignore, ignore_index, g, partial, P,
-                           loss, grad);
-    } else {
-      if (fuse)
-        hipLaunchKernelGGL((ce_grad<int32_t, true>), dim3(blocks), dim3(256), 0, s, logits,
-                           (const int32_t*)target, R, C, has_ignore, ignore_index, g, partial, P,
-                           loss, grad);
-      else
-        hipLaunchKernelGGL((ce_grad<int32_t, false>), dim3(blocks), dim3(256), 0, s, logits,
-                           (const int32_t*)target, R, C, has_ignore, ignore_index, g, partial, P,
-                           loss, grad);
-    }
-  }
   return hipGetLastError();
 }
 

@@ -1,0 +1,81 @@
+"""Index cross-entropy at the edges of its kernels' widths: the largest and smallest row of each
+form (one wave a row up to 1024 classes, one workgroup a row, the streamed form beyond), rows whose
+start is not 16-byte aligned, and sample counts formed in the kernel and by the launch before."""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from synaptik_amd.program import ProgramBuilder
+from tests.gpu_helpers import run_program
+
+pytestmark = pytest.mark.gpu
+
+WIDTHS = [1, 64, 65, 513, 1024, 1025, 2044, 2045, 4093, 8188, 8189, 16380, 16381, 32764, 32767,
+          65532, 65535, 70001]
+
+
+@pytest.mark.parametrize("ignore", [None, -100])
+@pytest.mark.parametrize("C", WIDTHS)
+def test_widths(ctx, C, ignore):
+    print(f"[index_ce] C={C} ignore={ignore}", flush=True)
+    R = 7
+    rng = np.random.default_rng(C)
+    logits = (rng.standard_normal((R, C)) * 3).astype(np.float32)
+    y = rng.integers(0, C, R)
+    y[0], y[1] = 0, C - 1
+    if ignore is not None:
+        y[2::3] = ignore
+    pb = ProgramBuilder()
+    sx, sy = pb.input(R * C), pb.input(R, "i64")
+    sl, sl2, sg = pb.output(1), pb.output(1), pb.output(R * C)
+    pb.index_ce(sx, sy, sl, R, C, grad=sg, ignore_index=ignore)
+    pb.index_ce(sx, sy, sl2, R, C, ignore_index=ignore)  # the loss alone
+    loss, loss2, grad = run_program(ctx, pb, [logits, y.astype(np.int64)], [sl, sl2, sg])
+    want = oracle.index_ce_mean(logits, y, ignore_index=ignore)
+    assert abs(loss[0] - want) <= 1e-5 * abs(want) + 1e-12
+    assert loss2[0] == loss[0]
+    np.testing.assert_allclose(grad.reshape(R, C),
+                               oracle.index_ce_grad(logits, y, ignore_index=ignore),
+                               rtol=1e-5, atol=1e-9)
+
+
+@pytest.mark.parametrize("R,C", [(4096, 18), (4097, 18), (1024, 1030), (1025, 1030)])
+def test_sample_count_of_many_rows(ctx, R, C):
+    print(f"[index_ce] R={R} C={C}", flush=True)
+    rng = np.random.default_rng(R)
+    logits = rng.standard_normal((R, C)).astype(np.float32)
+    y = rng.integers(0, C, R)
+    y[rng.random(R) < 0.3] = -1
+    pb = ProgramBuilder()
+    sx, sy = pb.input(R * C), pb.input(R, "i32")
+    sl, sg = pb.output(1), pb.output(R * C)
+    pb.index_ce(sx, sy, sl, R, C, grad=sg, ignore_index=-1)
+    loss, grad = run_program(ctx, pb, [logits, y.astype(np.int32)], [sl, sg])
+    want = oracle.index_ce_mean(logits, y, ignore_index=-1)
+    assert abs(loss[0] - want) <= 1e-5 * abs(want)
+    np.testing.assert_allclose(grad.reshape(R, C), oracle.index_ce_grad(logits, y, ignore_index=-1),
+                               rtol=1e-5, atol=1e-9)
+
+
+def test_special_rows(ctx):
+    """NaN and infinite logits and a row of nothing but -inf, on both row forms."""
+    for C in (70, 1500):
+        rng = np.random.default_rng(C)
+        logits = rng.standard_normal((6, C)).astype(np.float32)
+        logits[0, 3] = np.nan
+        logits[1, 4] = np.inf
+        logits[2, :] = -np.inf
+        logits[3, 5] = -np.inf
+        logits[4, :] = -0.0
+        y = np.array([3, 5, 1, 7, 0, 2])
+        pb = ProgramBuilder()
+        sx, sy = pb.input(6 * C), pb.input(6, "i64")
+        sl, sg = pb.output(1), pb.output(6 * C)
+        pb.index_ce(sx, sy, sl, 6, C, grad=sg)
+        loss, grad = run_program(ctx, pb, [logits, y.astype(np.int64)], [sl, sg])
+        want = oracle.index_ce_grad(logits, y)
+        got = grad.reshape(6, C)
+        assert np.isnan(loss[0])
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        fin = ~np.isnan(want)
+        np.testing.assert_allclose(got[fin], want[fin], rtol=1e-5, atol=1e-9)
