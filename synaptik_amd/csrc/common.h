@@ -71,6 +71,9 @@ __device__ __forceinline__ float java_max(float a, float b) {
 // Streaming (non-temporal) 16-byte loads and stores for data touched once per kernel: they do
 // not displace cache lines other work still needs, which lifts the large row kernels' HBM rate.
 typedef float float4v __attribute__((ext_vector_type(4)));
+// A 16-byte vector that may sit at any float: the hardware's vector loads and stores take such
+// addresses.
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ float4 ld_stream(const float4* a) {
   const float4v t = __builtin_nontemporal_load(reinterpret_cast<const float4v*>(a));
   return make_float4(t[0], t[1], t[2], t[3]);

@@ -10,24 +10,11 @@
 // which is what the matrix cores do; results differ from the sequential no-FMA CPU oracle only
 // by reduction order (and are bit-identical when all partial sums are exact).
 //
-// Design (one workgroup per BM x BN output tile):
-//   * v_mfma_f32_32x32x2_f32: each wave owns a WM x WN sub-tile as (WM/32) x (WN/32)
-//     32x32 accumulator blocks (16 fp32 accumulators per lane per block).
-//   * Both operand tiles are staged through LDS in a [k][m] / [k][n] layout (m/n contiguous,
-//     padded pitch) so that every MFMA operand fetch is one conflict-light ds_read_b32 with
-//     consecutive lanes on consecutive addresses; K-contiguous global operands are transposed
-//     on the way in, M/N-contiguous ones are stored with ds_write_b128.
-//   * LDS is double buffered: the global loads of tile k+1 are issued into registers before the
-//     MFMAs of tile k, and written to the other LDS buffer afterwards (one barrier per tile).
-//   * Workgroup ids are remapped so that each of the 8 XCDs receives a contiguous, M-grouped
-//     block of output tiles: tiles that share A row-panels and B column-panels share an L2.
-//
-// The tile kernel lives in gemm_tile.h and is instantiated per operand layout in gemm_nn.hip,
-// gemm_nt.hip, gemm_tn.hip and gemm_tt.hip; this file holds the dispatch, the deterministic
-// split-K reduction and the K == 1 outer product.
+// Kernels: gemm_v2.h (operands copied straight into LDS: large aligned problems), gemm_direct.h
+// (operands loaded straight into registers: unaligned and small problems), gemm_skinny.hip (one
+// extent of at most 16). This file holds the dispatch between them, split-K and K == 1.
 #include "gemm_skinny.h"
 #include "gemm_tile.h"
-#include "gemm_v2.h"
 #include <algorithm>
 
 namespace shk {
@@ -208,29 +195,44 @@ hipError_t launch_tiles(const GemmParams& p, bool va, bool vb, bool split, hipSt
 }  // namespace
 
 namespace {
-// Split-K plan for problems too small to give every CU a 128x128 tile: slices of at least 128 of
-// K, enough of them to reach ~256 workgroups, at most 16.
-int64_t splitk_slices(int64_t M, int64_t N, int64_t K) {
-  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-  if (K < 512 || tiles >= 128) return 1;
-  int64_t s = (256 + tiles - 1) / tiles;
-  s = std::min<int64_t>(s, 16);
-  s = std::min<int64_t>(s, K / 128);
-  return std::max<int64_t>(s, 1);
+// Split-K plan: how many slices of K a problem with too few tiles for the chip is cut into (1:
+// none), at most 16 and of at least 128 of K. Figures: us on MI355X, the reduction pass included.
+//   * From 256 64x64 tiles on only K > 2048 is split, to reach 256 128x128 tiles: 1024x1024x8192 TN
+//     128.4 in four against 133.6 whole on 64x64 tiles.
+//   * Deep problems below that: as many slices as 256 workgroups of 64x64 tiles hold
+//     (64x4096x4096 26.6 in four against 33.3 whole on 32x32 tiles; TN 512x256x8192 26.3 in eight,
+//     600x600x4000 44.0 in two against 60). Deep is K >= 1024 when an operand is M/N-contiguous,
+//     whose 32x32 tiles read poorly (512x1024x1024 TN 16.7 against 56.7), K >= 2048 and 32 tiles
+//     otherwise (K >= 1024 for 128 tiles or more: 512x1024x1024 16.7 against 19.2).
+//   * The others run on 32x32 tiles whose workgroups split K among their waves; slices only up to
+//     192 workgroups (32x1024x1024 8.1 in six against 11.2; 128x1024x512 7.9 whole against 8.4).
+// `nt`: both operands K-contiguous.
+int64_t gemm_slices(int64_t M, int64_t N, int64_t K, bool nt) {
+  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
+  const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64);
+  const int64_t t32 = ((M + 31) / 32) * ((N + 31) / 32);
+  if (K < 512 || t128 >= 128) return 1;
+  int64_t s;
+  if (t64 >= 256) s = K <= 2048 ? 1 : (256 + t128 - 1) / t128;
+  else if (nt ? (K >= 2048 && t64 >= 32) || (K >= 1024 && t64 >= 128) : K >= 1024) s = 256 / t64;
+  else s = 192 / t32;
+  return std::max<int64_t>(1, std::min<int64_t>(s, std::min<int64_t>(16, K / 128)));
+}
+int64_t gemm_slices(const GemmParams& p) {
+  return p.K > 1 ? gemm_slices(p.M, p.N, p.K, !p.transA && p.transB) : 1;
 }
 int64_t splitk_chunk(int64_t K, int64_t s) {
   const int64_t c = (K + s - 1) / s;
-  return ((c + 31) / 32) * 32;  // whole k-tiles of either tile kernel (BK 16 or 32) per slice
+  return ((c + 31) / 32) * 32;  // whole k-tiles of either kernel (16 or 32 deep) per slice
 }
 }  // namespace
 
 int64_t gemm_workspace_floats(int64_t M, int64_t N, int64_t K, bool colsum) {
   if (M <= 0 || N <= 0) return 0;
   int64_t floats = 0;
-  const int64_t s = K > 1 ? splitk_slices(M, N, K) : 1;
-  if (s > 1) {
-    const int64_t slices = (K + splitk_chunk(K, s) - 1) / splitk_chunk(K, s);
-    floats = slices * M * N;
+  if (K > 1) {  // of the operand layout that needs more
+    const int64_t s = std::max(gemm_slices(M, N, K, false), gemm_slices(M, N, K, true));
+    if (s > 1) floats = (K + splitk_chunk(K, s) - 1) / splitk_chunk(K, s) * M * N;
   }
   floats = std::max<int64_t>(floats, skinny_workspace_floats(M, N, K));
   if (colsum && K >= 2 && K <= 16)  // small-K kernel: one binary64 partial row per row block
@@ -252,16 +254,9 @@ void vector_operands(const GemmParams& p, bool& va, bool& vb) {
   va = a_contig % 4 == 0 && p.lda % 4 == 0 && aligned16(p.A);
   vb = b_contig % 4 == 0 && p.ldb % 4 == 0 && aligned16(p.B);
 }
-// Whether this GEMM is split along K: problems with too few 128x128 tiles are, unless the
-// direct-to-LDS kernel can run them whole on 64x64 tiles (no partials, no reduction pass).
-bool use_split(const GemmParams& in, bool have_workspace) {
-  if (!have_workspace || in.K <= 1 || splitk_slices(in.M, in.N, in.K) <= 1) return false;
-  GemmParams p = in;
-  p.kchunk = 0;
-  p.partial = nullptr;
-  bool va, vb;
-  vector_operands(p, va, vb);
-  return !(v2_enabled() && v2_choose(p, va, vb) == 64);
+// Whether this GEMM is split along K.
+bool use_split(const GemmParams& p, bool have_workspace) {
+  return have_workspace && gemm_slices(p) > 1;
 }
 }  // namespace
 
@@ -320,7 +315,7 @@ hipError_t launch_gemm_core(const GemmParams& in, float* workspace, hipStream_t 
   if (route != SKINNY_NONE && (route != SKINNY_COL_OUTER || workspace != nullptr))
     return launch_skinny(p, route, workspace, s);
   if (use_split(p, workspace != nullptr)) {
-    p.kchunk = splitk_chunk(p.K, splitk_slices(p.M, p.N, p.K));
+    p.kchunk = splitk_chunk(p.K, gemm_slices(p));
     const int slices = (int)((p.K + p.kchunk - 1) / p.kchunk);
     p.partial = workspace;
     bool va, vb;

@@ -2,11 +2,17 @@
 // BK = 32, four waves of (BT/2) x (BT/2), v_mfma_f32_16x16x4_f32, operands moved from HBM straight
 // into LDS.
 //
-// Used when both operands allow 16-byte loads, K and N are multiples of 4 and the problem gives
-// enough workgroups (see v2_choose); ragged M / N / K edges are handled by the TAIL variants.
-// Every other case runs the register-staged kernel in gemm_tile.h. The epilogues are the same:
-// bias + activation, activation gradient, accumulate, the binary64 column-sum partials of a bias
-// gradient, and the staged optimizer update of a weight gradient.
+// Used wherever the problem gives enough workgroups (see v2_choose). Ragged M / N / K edges are
+// handled by the TAIL variants when both operands allow aligned 16-byte loads and K and N are
+// multiples of 4, and by the U variants otherwise; gemm_direct.h runs the problems with too few
+// tiles. The epilogues are the same: bias + activation, activation gradient, accumulate, the
+// binary64 column-sum partials of a bias gradient, and the staged optimizer update of a weight
+// gradient.
+//
+// U, before (a register-staged kernel with 4-byte loads) and after, us on MI355X: 3001x2047x1531 NT
+// 267 -> 162, 3001x1531x2047 NN 356 -> 182, 2047x1531x3001 TN 219 -> 155; 4095^3 1038 / 1012 / 1020
+// (132 to 136 TFLOP/s; aligned 4096^3: 147). Four-byte copies into LDS instead, which need no
+// moved tile and no cut chunk, took 198 / 246 / 236.
 //
 // Data movement:
 //   * global_load_lds_dwordx4: each lane copies 16 bytes from HBM to LDS without passing through
@@ -44,7 +50,12 @@ constexpr int V2_BK = 32, V2_NT = 256;
 // than with four).
 constexpr int V2_GROUP = 4, V2_GROUP64 = 2;
 
-template <int BT>
+// U (unaligned): operands of any alignment, leading dimension, K, M and N. A 16-byte copy may start
+// at any float of the operand; what it may not do is take in floats beyond the operand's row, so
+//   * the last tile of an M/N-contiguous operand is moved back to end with the operand (its extent
+//     is at least BT) and the epilogue leaves out the rows or columns the tile before it stores;
+//   * the chunk of a K-contiguous row that K cuts is loaded float by float (once per tile).
+template <int BT, bool U>
 struct V2Cfg {
   static constexpr int NB = BT / 32;      // 16x16 blocks per wave and dimension
   static constexpr int WT = BT / 2;       // wave tile edge
@@ -59,9 +70,9 @@ struct V2Cfg {
 
 // Per-lane source offsets (bytes, relative to the tile origin) of the NI 16-byte copies this
 // thread issues per operand per k-tile, where they land, and (TAIL) the chunk's coordinates.
-template <bool KMAJ, int BT, bool TAIL>
+template <bool KMAJ, int BT, bool TAIL, bool U>
 struct V2Loader {
-  using Cfg = V2Cfg<BT>;
+  using Cfg = V2Cfg<BT, U>;
   uint32_t voff[Cfg::NI];
   int vrow[Cfg::NI], vk[Cfg::NI];  // first row (M/N) and first k of the chunk in the tile
   uint32_t wdst;                   // this wave's byte offset inside a stage (wave-uniform)
@@ -96,14 +107,22 @@ struct V2Loader {
     const uint32_t dst =
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)lds + I * 4096u + wdst;
     // a whole tile row-range and a whole k-tile (uniform) need no per-lane bounds
-    if (!TAIL || (rows_left >= BT && k_left >= V2_BK) || (vrow[I] < rows_left && vk[I] < k_left)) {
+    if (!TAIL || (rows_left >= BT && k_left >= V2_BK) ||
+        (vrow[I] < rows_left && vk[I] + (U && KMAJ ? 3 : 0) < k_left)) {
       asm volatile("global_load_lds_dwordx4 %0, %1"
                    :
                    : "v"(voff[I]), "s"(tile), "{m0}"(dst)
                    : "memory");
     } else {
       const int w = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
-      *reinterpret_cast<floatx4*>(lds + (I * 4 + w) * 256 + lane * 4) = floatx4{0.f, 0.f, 0.f, 0.f};
+      floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
+      if (U && KMAJ && vrow[I] < rows_left && vk[I] < k_left) {  // the chunk that K cuts
+        const float* src = tile + voff[I] / 4;
+        v[0] = src[0];
+        if (vk[I] + 1 < k_left) v[1] = src[1];
+        if (vk[I] + 2 < k_left) v[2] = src[2];
+      }
+      *reinterpret_cast<floatx4*>(lds + (I * 4 + w) * 256 + lane * 4) = v;
     }
   }
 };
@@ -125,7 +144,7 @@ struct V2Loader {
 // the accumulators back through the same interleave (v2_row / v2_col).
 template <bool KMAJ, int BT>
 struct V2Frag {
-  static constexpr int NB = V2Cfg<BT>::NB;
+  static constexpr int NB = V2Cfg<BT, false>::NB;
   static constexpr int ITEMS = KMAJ ? NB : 4;  // fragment reads per half
   floatx4 f[NB];
   template <int H, int T>
@@ -171,6 +190,38 @@ struct V2ReadOrder {
   }
 };
 
+// A lane's segment of four consecutive columns of a result row: 16-byte accesses; with U at any
+// float address, and element by element where not all of columns lo .. hi - 1 are the lane's.
+template <bool U>
+struct V2Segment {
+  int lo, hi;
+  __device__ __forceinline__ bool holds(int c) const { return !U || (c >= lo && c < hi); }
+  __device__ __forceinline__ bool whole() const { return lo == 0 && hi >= 4; }
+  __device__ __forceinline__ floatx4 load(const float* src) const {
+    if constexpr (!U) return *reinterpret_cast<const floatx4*>(src);
+    if (whole()) {
+      const float4u v = *reinterpret_cast<const float4u*>(src);
+      return floatx4{v[0], v[1], v[2], v[3]};
+    }
+    floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (holds(c)) v[c] = src[c];
+    return v;
+  }
+  __device__ __forceinline__ void store(float* dst, const floatx4& v) const {
+    if constexpr (!U) {
+      *reinterpret_cast<floatx4*>(dst) = v;
+    } else if (whole()) {
+      *reinterpret_cast<float4u*>(dst) = float4u{v[0], v[1], v[2], v[3]};
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (holds(c)) dst[c] = v[c];
+    }
+  }
+};
+
 __device__ __forceinline__ void v2_wait_all() {
   // vmcnt(0) and lgkmcnt(0): this wave's LDS copies have landed and its LDS reads returned
   __builtin_amdgcn_s_waitcnt(0x0070);
@@ -190,10 +241,11 @@ __device__ __forceinline__ void v2_barrier() {
 // in LDS and share the epilogue, each value the sum group 0 + group 1 (a fixed order), stored as
 // the result or, for a slice, as the slice's partial. It gives each SIMD two waves on problems
 // with too few tiles for two workgroups per CU, without more partials in HBM or a second launch.
-template <bool KA, bool KB, int BT, bool TAIL, int KS>
+template <bool KA, bool KB, int BT, bool TAIL, int KS, bool U = false>
 __global__ void __launch_bounds__(V2_NT * KS) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_f32_v2(GemmParams p) {
-  using Cfg = V2Cfg<BT>;
+  static_assert(!U || TAIL, "operands of any alignment have edges");
+  using Cfg = V2Cfg<BT, U>;
   constexpr int NB = Cfg::NB, WT = Cfg::WT, TILEF = Cfg::TILEF, NI = Cfg::NI, NG = Cfg::NG;
   __shared__ __attribute__((aligned(16))) float As0g[KS * TILEF];
   __shared__ __attribute__((aligned(16))) float Bs0g[KS * TILEF];
@@ -209,7 +261,10 @@ gemm_f32_v2(GemmParams p) {
   const int tilesM = (int)((p.M + BT - 1) / BT), tilesN = (int)((p.N + BT - 1) / BT);
   int tm, tn;
   tile_of(blockIdx.x, tilesM, tilesN, tm, tn);
-  const int64_t m0 = (int64_t)tm * BT, n0 = (int64_t)tn * BT;
+  // first row and column this tile stores, and its origin (U: moved back at the operand's end)
+  const int64_t m_first = (int64_t)tm * BT, n_first = (int64_t)tn * BT;
+  const int64_t m0 = U && !KA ? std::min<int64_t>(m_first, p.M - BT) : m_first;
+  const int64_t n0 = U && !KB ? std::min<int64_t>(n_first, p.N - BT) : n_first;
   const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, g = lane >> 4;
@@ -232,8 +287,8 @@ gemm_f32_v2(GemmParams p) {
   const float* b_tile = KB ? p.B + n0 * p.ldb + k_begin : p.B + n0 + k_begin * p.ldb;
   const int64_t a_step = KA ? V2_BK : V2_BK * p.lda;
   const int64_t b_step = KB ? V2_BK : V2_BK * p.ldb;
-  V2Loader<KA, BT, TAIL> la;
-  V2Loader<KB, BT, TAIL> lb;
+  V2Loader<KA, BT, TAIL, U> la;
+  V2Loader<KB, BT, TAIL, U> lb;
   la.init(p.lda);
   lb.init(p.ldb);
 
@@ -275,8 +330,9 @@ gemm_f32_v2(GemmParams p) {
   // i = (n % NB^2) / NB, j = n % NB, or i and j exchanged for a K-contiguous B); after each group, side(q) issues that group's share of the
   // LDS reads and copies. The scheduling barriers keep this order: reads and copies spread over
   // the MFMA stream instead of stalling it in one place.
-  auto mfma_half = [&](const V2Frag<KA, BT>& fa, const V2Frag<KB, BT>& fb, auto side) {
-    static_for<NG>([&](auto q) {
+  auto mfma_half = [&](const V2Frag<KA, BT>& fa, const V2Frag<KB, BT>& fb, auto side)
+      __attribute__((always_inline)) {
+    static_for<NG>([&](auto q) __attribute__((always_inline)) {
       constexpr int Q = decltype(q)::value;
       static_for<Cfg::GS>([&](auto u) {
         constexpr int N = Cfg::GS * Q + decltype(u)::value;
@@ -301,7 +357,7 @@ gemm_f32_v2(GemmParams p) {
   constexpr V2ReadOrder<KA, KB, NB> kOrder{};
   constexpr int NREAD = kOrder.N, RPG = (NREAD + NG / 2 - 1) / (NG / 2);
   auto read_item = [&](auto t, V2Frag<KA, BT>& fa, V2Frag<KB, BT>& fb, const float* As,
-                       const float* Bs, auto h) {
+                       const float* Bs, auto h) __attribute__((always_inline)) {
     constexpr int T = decltype(t)::value, H = decltype(h)::value;
     if constexpr (T < NREAD) {
       if constexpr (kOrder.op[T] == 0) fa.template load_item<H, kOrder.idx[T]>(As, a_base[H]);
@@ -309,13 +365,17 @@ gemm_f32_v2(GemmParams p) {
     }
   };
   // Copies of a k-tile: item c (c < 2 NI) is operand c % 2, instruction c / 2.
-  auto copy_item = [&](auto c, const float* at, const float* bt, float* As, float* Bs, int k_left) {
+  // (the pipeline's lambdas are inlined by force: a call would pass the tile origins, which the
+  // copies need in scalar registers, in vector registers)
+  auto copy_item = [&](auto c, const float* at, const float* bt, float* As, float* Bs, int k_left)
+      __attribute__((always_inline)) {
     constexpr int C = decltype(c)::value;
     if constexpr (C % 2 == 0) la.template issue<C / 2>(at, As, rows_a, k_left);
     else lb.template issue<C / 2>(bt, Bs, rows_b, k_left);
   };
-  auto copy_all = [&](const float* at, const float* bt, float* As, float* Bs, int k_left) {
-    static_for<2 * NI>([&](auto c) { copy_item(c, at, bt, As, Bs, k_left); });
+  auto copy_all = [&](const float* at, const float* bt, float* As, float* Bs, int k_left)
+      __attribute__((always_inline)) {
+    static_for<2 * NI>([&](auto c) __attribute__((always_inline)) { copy_item(c, at, bt, As, Bs, k_left); });
   };
 
   // Software pipeline over k-tiles (tile kt lives in stage kt % 2; fa0 / fb0 hold its first-half
@@ -338,7 +398,7 @@ gemm_f32_v2(GemmParams p) {
     if (TAIL && !(rows_a == BT && rows_b == BT && k_len >= 2 * V2_BK)) {
       v2_wait_all();
     } else {
-      if constexpr (NI == 4) __builtin_amdgcn_s_waitcnt(0x0F78);
+      if constexpr (BT == 128) __builtin_amdgcn_s_waitcnt(0x0F78);
       else __builtin_amdgcn_s_waitcnt(0x0F74);
     }
   } else {
@@ -347,7 +407,7 @@ gemm_f32_v2(GemmParams p) {
   v2_barrier();
   fa0.template load<0>(As0, a_base[0]);
   fb0.template load<0>(Bs0, b_base[0]);
-  auto step = [&](auto cur, int kt) {
+  auto step = [&](auto cur, int kt) __attribute__((always_inline)) {
     constexpr int CUR = decltype(cur)::value;
     float* Acur = CUR ? As1 : As0;
     float* Bcur = CUR ? Bs1 : Bs0;
@@ -358,7 +418,7 @@ gemm_f32_v2(GemmParams p) {
     const float* bt = b_tile + (int64_t)(kt + 2) * b_step;
     const int k_left = (int)(k_len - (int64_t)(kt + 2) * V2_BK);
     __builtin_amdgcn_sched_barrier(0);
-    mfma_half(fa0, fb0, [&](auto q) {
+    mfma_half(fa0, fb0, [&](auto q) __attribute__((always_inline)) {
       constexpr int Q = decltype(q)::value;
       if constexpr (Q < NG / 2) {
         static_for<RPG>([&](auto r) {
@@ -372,7 +432,7 @@ gemm_f32_v2(GemmParams p) {
       v2_barrier();
     }
     __builtin_amdgcn_sched_barrier(0);
-    mfma_half(fa1, fb1, [&](auto q) {
+    mfma_half(fa1, fb1, [&](auto q) __attribute__((always_inline)) {
       constexpr int Q = decltype(q)::value;
       if constexpr (Q < NG / 2) {
         if (more) {
@@ -383,7 +443,7 @@ gemm_f32_v2(GemmParams p) {
         }
       } else {
         if (copy) {
-          static_for<Cfg::CPG>([&](auto c) {
+          static_for<Cfg::CPG>([&](auto c) __attribute__((always_inline)) {
             copy_item(std::integral_constant<int, (Q - NG / 2) * Cfg::CPG + decltype(c)::value>{},
                       at, bt, Acur, Bcur, k_left);
           });
@@ -414,7 +474,8 @@ gemm_f32_v2(GemmParams p) {
           constexpr int R = decltype(r)::value;
           const int64_t row = m0 + wm * WT + v2_row(I, R);
           const int64_t col = n0 + wn * WT + v2_col(J, R);
-          if (!TAIL || (row < p.M && col < p.N)) part[row * p.N + col] = acc[I][J][R];
+          if (!TAIL || (row < p.M && col < p.N && (!U || (row >= m_first && col >= n_first))))
+            part[row * p.N + col] = acc[I][J][R];
         });
       });
     });
@@ -480,7 +541,12 @@ gemm_f32_v2(GemmParams p) {
   static_assert(TSTEPS % EPI_CH == 0, "whole chunks");
   const int tfirst = kgroup * TSTEPS;
   const int64_t row_e = m0 + wm * WT + rg, col_e = n0 + wn * WT + 4 * q;
-  const bool col_ok = !TAIL || col_e < p.N;  // N is a multiple of 4: whole segments
+  // U: any N, and columns the tile before stores, so a lane's segment may be partial; otherwise N
+  // is a multiple of 4
+  const V2Segment<U> seg{(int)std::max<int64_t>(0, n_first - col_e),
+                         (int)std::min<int64_t>(4, p.N - col_e)};
+  const bool col_ok = !TAIL || (U ? seg.lo < seg.hi : col_e < p.N);
+  auto row_out = [&](int64_t row) { return TAIL && (!col_ok || row >= p.M || (U && row < m_first)); };
   if constexpr (KS == 2) {
     if (p.partial != nullptr) {
       // split-K slice of a KS = 2 workgroup: the slice's partial sums (group 0's + group 1's),
@@ -488,8 +554,8 @@ gemm_f32_v2(GemmParams p) {
       float* part = p.partial + (int64_t)blockIdx.y * p.M * p.N;
       for (int t = tfirst; t < tfirst + TSTEPS; ++t) {
         const int64_t row = row_e + RSTEP * t;
-        if (TAIL && (!col_ok || row >= p.M)) continue;
-        *reinterpret_cast<floatx4*>(part + row * p.N + col_e) = tile_row(t);
+        if (row_out(row)) continue;
+        seg.store(part + row * p.N + col_e, tile_row(t));
       }
       return;
     }
@@ -510,32 +576,33 @@ gemm_f32_v2(GemmParams p) {
         static_for<EPI_CH>([&](auto ic) {
           constexpr int I = decltype(ic)::value;
           const int64_t row = row_e + RSTEP * (t0 + I);
-          const bool in = !TAIL || (col_ok && row < p.M);
+          const bool in = !row_out(row);
           const int64_t e = row * p.N + col_e;
           const floatx4 z = floatx4{0.f, 0.f, 0.f, 0.f};
-          pv[I] = in ? *reinterpret_cast<const floatx4*>(u.p + e) : z;
-          mv[I] = in && u.m != nullptr ? *reinterpret_cast<const floatx4*>(u.m + e) : z;
-          vv[I] = !SGD && in ? *reinterpret_cast<const floatx4*>(u.v + e) : z;
+          pv[I] = in ? seg.load(u.p + e) : z;
+          mv[I] = in && u.m != nullptr ? seg.load(u.m + e) : z;
+          vv[I] = !SGD && in ? seg.load(u.v + e) : z;
         });
         static_for<EPI_CH>([&](auto ic) {
           constexpr int I = decltype(ic)::value;
           const int64_t row = row_e + RSTEP * (t0 + I);
-          if (TAIL && (!col_ok || row >= p.M)) return;
+          if (row_out(row)) return;
           const int64_t e = row * p.N + col_e;
           const floatx4 gv = tile_row(t0 + I);
           floatx4 pc, mc, vc = floatx4{0.f, 0.f, 0.f, 0.f};
           static_for<4>([&](auto c) {
             constexpr int C = decltype(c)::value;
-            float pe, me, ve = 0.0f;
-            if constexpr (SGD) sgd_element(u, uc.first, pv[I][C], gv[C], mv[I][C], pe, me, chk);
-            else adam_element(u, uc.k, pv[I][C], gv[C], mv[I][C], vv[I][C], pe, me, ve, chk);
+            float pe, me, ve = 0.0f, ce = chk;
+            if constexpr (SGD) sgd_element(u, uc.first, pv[I][C], gv[C], mv[I][C], pe, me, ce);
+            else adam_element(u, uc.k, pv[I][C], gv[C], mv[I][C], vv[I][C], pe, me, ve, ce);
+            if (seg.holds(C)) chk = ce;
             pc[C] = pe;
             mc[C] = me;
             vc[C] = ve;
           });
-          *reinterpret_cast<floatx4*>(u.pn + e) = pc;
-          if (u.mn != nullptr) *reinterpret_cast<floatx4*>(u.mn + e) = mc;
-          if constexpr (!SGD) *reinterpret_cast<floatx4*>(u.vn + e) = vc;
+          seg.store(u.pn + e, pc);
+          if (u.mn != nullptr) seg.store(u.mn + e, mc);
+          if constexpr (!SGD) seg.store(u.vn + e, vc);
         });
       }
     };
@@ -546,7 +613,7 @@ gemm_f32_v2(GemmParams p) {
   }
   const bool has_bias = p.bias != nullptr;
   floatx4 bias = floatx4{0.f, 0.f, 0.f, 0.f};
-  if (has_bias && col_ok) bias = *reinterpret_cast<const floatx4*>(p.bias + col_e);
+  if (has_bias && col_ok) bias = seg.load(p.bias + col_e);
   double cs[4] = {0.0, 0.0, 0.0, 0.0};  // fused column sums of this lane's stored values
   auto store_rows = [&](auto modec, auto actc, auto accc) {
     constexpr int MODE = decltype(modec)::value, ACT = decltype(actc)::value;
@@ -563,8 +630,8 @@ gemm_f32_v2(GemmParams p) {
         static_for<SCH>([&](auto ic) {
           constexpr int I = decltype(ic)::value;
           const int64_t row = row_e + RSTEP * (t0 + I);
-          ya[I] = (!TAIL || (col_ok && row < p.M))
-                      ? *reinterpret_cast<const floatx4*>(p.aux + row * p.ldaux + col_e)
+          ya[I] = !row_out(row)
+                      ? seg.load(p.aux + row * p.ldaux + col_e)
                       : floatx4{0.f, 0.f, 0.f, 0.f};
         });
       }
@@ -572,7 +639,7 @@ gemm_f32_v2(GemmParams p) {
         constexpr int I = decltype(ic)::value;
         const int t = t0 + I;
         const int64_t row = row_e + RSTEP * t;
-        if (TAIL && (!col_ok || row >= p.M)) return;
+        if (row_out(row)) return;
         floatx4 v = tile_row(t);
         if constexpr (MODE != 1) {
           if (has_bias) v = floatx4{v[0] + bias[0], v[1] + bias[1], v[2] + bias[2], v[3] + bias[3]};
@@ -584,12 +651,12 @@ gemm_f32_v2(GemmParams p) {
             v[C] = act_grad(ACT, v[C], y[C]);
           });
         }
-        floatx4* dst = reinterpret_cast<floatx4*>(p.C + row * p.ldc + col_e);
-        if constexpr (ACC) {
-          const floatx4 o = *dst;
+        float* dst = p.C + row * p.ldc + col_e;
+        if (U ? p.accumulate != 0 : ACC) {
+          const floatx4 o = seg.load(dst);
           v = floatx4{o[0] + v[0], o[1] + v[1], o[2] + v[2], o[3] + v[3]};
         }
-        *dst = v;
+        seg.store(dst, v);
         if constexpr (MODE == 2) {
           // the cotangent of the activation input from the stored activation and dY
           const floatx4 gy = ya[I];
@@ -597,14 +664,14 @@ gemm_f32_v2(GemmParams p) {
             constexpr int C = decltype(c)::value;
             v[C] = act_grad(ACT, gy[C], v[C]);
           });
-          *reinterpret_cast<floatx4*>(p.dz + row * p.ldaux + col_e) = v;
+          seg.store(p.dz + row * p.ldaux + col_e, v);
         }
         static_for<4>([&](auto c) { cs[decltype(c)::value] += (double)v[decltype(c)::value]; });
       });
     }
   };
   auto by_acc = [&](auto modec, auto actc) {
-    if (p.accumulate) store_rows(modec, actc, std::true_type{});
+    if (!U && p.accumulate) store_rows(modec, actc, std::bool_constant<!U>{});
     else store_rows(modec, actc, std::false_type{});
   };
   auto by_act = [&](auto modec) {
@@ -627,7 +694,9 @@ gemm_f32_v2(GemmParams p) {
     if (rg == 0 && col_ok) {
       // one partial row per wave row and K group
       double* dst = p.colsum_partial + (((int64_t)tm * 2 + wm) * KS + kgroup) * p.N + col_e;
-      static_for<4>([&](auto c) { dst[decltype(c)::value] = cs[decltype(c)::value]; });
+      static_for<4>([&](auto c) {
+        if (seg.holds(decltype(c)::value)) dst[decltype(c)::value] = cs[decltype(c)::value];
+      });
     }
   }
 }
@@ -650,28 +719,42 @@ inline bool v2_ks2_enabled() {
   return on;
 }
 
-// Kernel choice for a GEMM (0: none, the register-staged kernel runs it; else the tile edge).
-//   * both operands allow 16-byte loads, K and N are multiples of 4 and, for the transposed
-//     epilogue, its pointers are 16-byte aligned with leading dimensions multiples of 4;
-//   * BT = 128 when there are at least 256 such tiles (times split-K slices);
-//   * BT = 64 for problems with at least 128 64x64 tiles and K <= 2048 that are not split, in
-//     place of splitting K (no partials, no reduction pass).
-// TAIL variants run when M, N or K (or the slice) is not a whole number of tiles.
-inline int v2_choose(const GemmParams& p, bool va, bool vb) {
-  if (!va || !vb || p.K % 4 != 0 || p.N % 4 != 0 || p.K < 4) return 0;
+// Whether both operands allow 16-byte copies and the epilogue whole, aligned 16-byte segments:
+// K and N multiples of 4 and, for the transposed epilogue, its pointers 16-byte aligned with
+// leading dimensions multiples of 4. Otherwise the kernel runs in its U form.
+inline bool v2_aligned(const GemmParams& p, bool va, bool vb) {
+  if (!va || !vb || p.K % 4 != 0 || p.N % 4 != 0) return false;
   auto al = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; };
-  if (p.kchunk > 0) {
-    if (p.kchunk % V2_BK != 0 || p.partial == nullptr) return 0;
-  } else if (p.upd.pn != nullptr) {
+  if (p.kchunk > 0) return al(p.partial);
+  if (p.upd.pn != nullptr) {
     const GemmUpdate& u = p.upd;
-    if (!al(u.p) || !al(u.pn) || (u.m != nullptr && (!al(u.m) || !al(u.mn))) ||
-        (u.kind != 0 && (!al(u.v) || !al(u.vn))))
-      return 0;
-  } else {
-    if (!al(p.C) || p.ldc % 4 != 0 || (p.bias != nullptr && !al(p.bias))) return 0;
-    if (p.mode != 0 && (!al(p.aux) || p.ldaux % 4 != 0)) return 0;
-    if (p.mode == 2 && !al(p.dz)) return 0;
+    return al(u.p) && al(u.pn) && (u.m == nullptr || (al(u.m) && al(u.mn))) &&
+           (u.kind == 0 || (al(u.v) && al(u.vn)));
   }
+  return al(p.C) && p.ldc % 4 == 0 && (p.bias == nullptr || al(p.bias)) &&
+         (p.mode == 0 || (al(p.aux) && p.ldaux % 4 == 0)) && (p.mode != 2 || al(p.dz));
+}
+
+// Tile edge of the direct-to-LDS kernel for a GEMM, or 0 when gemm_direct runs it. Figures: us on
+// MI355X for one GEMM, sizes M x N x K.
+//   * Whole K. A CU works through its 128x128 tiles two at a time, so the time goes with
+//     ceil(tiles / 256) of them: 384 tiles take as long as 512. 64x64 tiles, a quarter of the
+//     work each, fill the last round four times finer and are otherwise about 2% slower. 128 when
+//     it needs no more of these quarter units: 3072x2048x1536 NT 177 (128) against 139 (64),
+//     5120x2048x1024 180 against 152, 4096x1536x1024 121 against 98; 4096x1024x1024 65.2 against
+//     65.9, 4095^3 1038 against 1068.
+//   * 64 needs 128 tiles; below that a workgroup of gemm_direct's 32x32 tiles finishes sooner
+//     (256x1024x1024 NT 11.6 against 18.9). With both operands K-contiguous and K < 1024 that
+//     holds for 128 tiles too (512x1024x400 10.1 against 13.0; NN 14.6 against 12.8).
+//   * Split-K slices (gemm_slices): 128 where the plan counted in 128x128 tiles, 64 for the other
+//     plans that reach 128 workgroups; gemm_direct for the rest.
+// TAIL variants run when M, N or K (or the slice) is not a whole number of tiles.
+inline int v2_choose(const GemmParams& p, bool aligned) {
+  // the moved last tile of the U form needs a whole tile of its operand
+  auto fits = [&](int bt) {
+    return aligned || ((!p.transA || p.M >= bt) && (p.transB || p.N >= bt));
+  };
+  if (p.K < 4 || (p.kchunk > 0 && (p.kchunk % V2_BK != 0 || p.partial == nullptr))) return 0;
   const int64_t ld = std::max(p.lda, p.ldb);
   if ((p.M + 128) * ld >= (1LL << 31) || (p.N + 128) * ld >= (1LL << 31) ||
       (p.K + 128) * ld >= (1LL << 31))
@@ -680,72 +763,61 @@ inline int v2_choose(const GemmParams& p, bool va, bool vb) {
   const int64_t t128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
   const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
   if (t64 >= (1LL << 31) || slices >= 65536) return 0;
-  if (t128 * slices >= 256) return 128;
-  if (p.kchunk == 0 && t64 >= 128 && p.K <= 2048) return 64;
-  return 0;
+  if (p.kchunk > 0) {
+    if (aligned && t64 >= 256 && t128 * slices >= 256) return 128;
+    return t64 * slices >= 128 && fits(64) ? 64 : 0;
+  }
+  if (t128 >= 256 && 4 * ((t128 + 255) / 256) <= (t64 + 255) / 256 && fits(128)) return 128;
+  if (t64 < 128 || !fits(64)) return 0;
+  return !p.transA && p.transB && p.K < 1024 && t64 == 128 ? 0 : 64;
 }
 
-// In-workgroup split-K (KS = 2) for 64x64 tiles: fewer than two tiles per CU and at least
-// eight k-tiles per group.
-inline bool v2_split_in_group(const GemmParams& p, int bt) {
-  const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
-  return v2_ks2_enabled() && bt == 64 && p.kchunk == 0 && t64 < 512 && p.K >= 16 * V2_BK;
+// In-workgroup split-K (KS = 2): fewer than two workgroups per CU and at least eight k-tiles per
+// group. Eight waves give each SIMD two, as two four-wave workgroups per CU would, without more
+// partials in HBM. 128x128 tiles only on split-K slices.
+inline bool v2_split_in_group(const GemmParams& p, int bt, int64_t tiles, int64_t slices) {
+  const int64_t span = p.kchunk > 0 ? p.kchunk : p.K;
+  return v2_ks2_enabled() && (bt == 64 || (p.kchunk > 0 && p.partial != nullptr)) &&
+         tiles * slices < 512 && span >= 16 * V2_BK;
 }
 
-// In-workgroup split-K (KS = 2) for the split-K slices of 128x128 tiles: at most one workgroup
-// per CU (fewer than 512 tile slices) and at least eight k-tiles per group. Eight waves give each
-// SIMD two, as two four-wave workgroups per CU would, without more slices in HBM.
-inline bool v2_split_slices_in_group(const GemmParams& p, unsigned tiles, unsigned slices) {
-  return v2_ks2_enabled() && p.kchunk > 0 && p.partial != nullptr &&
-         (int64_t)tiles * slices < 512 && p.kchunk >= 16 * V2_BK;
-}
-
-template <bool TA, bool TB, int BT>
+template <bool TA, bool TB, int BT, bool U>
 hipError_t launch_v2_bt(const GemmParams& p, hipStream_t s) {
-  g_colsum_rows = ((p.M + BT - 1) / BT) * 2;
   const unsigned tiles = (unsigned)(((p.M + BT - 1) / BT) * ((p.N + BT - 1) / BT));
   const unsigned slices = p.kchunk > 0 ? (unsigned)((p.K + p.kchunk - 1) / p.kchunk) : 1u;
   const int64_t span = p.kchunk > 0 ? p.kchunk : p.K;
-  if constexpr (BT == 64) {
-    if (v2_split_in_group(p, BT)) {
-      g_colsum_rows = ((p.M + BT - 1) / BT) * 4;  // per wave row and K group
-      // both groups whole k-tiles only when K is a multiple of 2 BK
-      const bool tail = p.M % BT != 0 || p.N % BT != 0 || p.K % (2 * V2_BK) != 0;
-      if (tail)
-        hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, true, 2>), dim3(tiles), dim3(2 * V2_NT), 0,
-                           s, p);
-      else
-        hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, false, 2>), dim3(tiles), dim3(2 * V2_NT), 0,
-                           s, p);
-      return hipGetLastError();
-    }
+  const bool ks2 = !(U && BT == 128) && v2_split_in_group(p, BT, tiles, slices);
+  g_colsum_rows = ((p.M + BT - 1) / BT) * (ks2 ? 4 : 2);  // per wave row and K group
+  const dim3 grid(tiles, slices), block(ks2 ? 2 * V2_NT : V2_NT);
+  if constexpr (U) {
+    if (BT == 64 && ks2)
+      hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, 64, true, 2, true>), grid, block, 0, s, p);
+    else
+      hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, true, 1, true>), grid, dim3(V2_NT), 0, s, p);
+    return hipGetLastError();
+  } else {
+    // whole tiles only when every slice's K range (with two groups, each half of it) is a whole
+    // number of k-tiles, the last slice's included
+    const int64_t unit = (ks2 ? 2 : 1) * V2_BK;
+    const bool tail = p.M % BT != 0 || p.N % BT != 0 || span % unit != 0 ||
+                      (p.K - (int64_t)(slices - 1) * span) % unit != 0;
+    if (ks2 && tail)
+      hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, true, 2>), grid, block, 0, s, p);
+    else if (ks2)
+      hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, false, 2>), grid, block, 0, s, p);
+    else if (tail)
+      hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, true, 1>), grid, block, 0, s, p);
+    else
+      hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, false, 1>), grid, block, 0, s, p);
+    return hipGetLastError();
   }
-  const bool tail = p.M % BT != 0 || p.N % BT != 0 || span % V2_BK != 0 || p.K % V2_BK != 0;
-  if constexpr (BT == 128) {
-    if (v2_split_slices_in_group(p, tiles, slices)) {
-      // both groups whole k-tiles of every slice only when every slice, the last included, is a
-      // multiple of 2 BK
-      const bool tail2 = tail || span % (2 * V2_BK) != 0 ||
-                         (p.K - (int64_t)(slices - 1) * span) % (2 * V2_BK) != 0;
-      if (tail2)
-        hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, true, 2>), dim3(tiles, slices),
-                           dim3(2 * V2_NT), 0, s, p);
-      else
-        hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, false, 2>), dim3(tiles, slices),
-                           dim3(2 * V2_NT), 0, s, p);
-      return hipGetLastError();
-    }
-  }
-  if (tail)
-    hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, true, 1>), dim3(tiles, slices), dim3(V2_NT), 0, s, p);
-  else
-    hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, BT, false, 1>), dim3(tiles, slices), dim3(V2_NT), 0, s, p);
-  return hipGetLastError();
 }
 
 template <bool TA, bool TB>
-hipError_t launch_v2(const GemmParams& p, int bt, hipStream_t s) {
-  return bt == 64 ? launch_v2_bt<TA, TB, 64>(p, s) : launch_v2_bt<TA, TB, 128>(p, s);
+hipError_t launch_v2(const GemmParams& p, int bt, bool aligned, hipStream_t s) {
+  if (bt == 64)
+    return aligned ? launch_v2_bt<TA, TB, 64, false>(p, s) : launch_v2_bt<TA, TB, 64, true>(p, s);
+  return aligned ? launch_v2_bt<TA, TB, 128, false>(p, s) : launch_v2_bt<TA, TB, 128, true>(p, s);
 }
 
 }  // namespace

@@ -8,10 +8,6 @@
 
 namespace shk {
 
-// A 16-byte vector that may sit at any float (the hardware takes such addresses; the row of
-// another tensor with the same ordinals need not share the alignment of the one read).
-typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
-
 struct RowGroups {
   int lead;    // floats of group 0 that precede the row
   int groups;  // groups that hold a float of the row
@@ -37,7 +33,8 @@ struct RowGroups {
     v.w = c + 3 < width ? row[c + 3] : fill;
     return v;
   }
-  // Writes group q to `row`, which may be another tensor's row of the same width.
+  // Writes group q to `row`, which may be another tensor's row of the same width (it need not
+  // share the alignment of the one read).
   __device__ __forceinline__ void store(float* row, int q, const float4& v) const {
     const int c = first(q);
     if (whole(q)) {
