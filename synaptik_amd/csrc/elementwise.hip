@@ -15,6 +15,7 @@
 // Java Math.max (NaN wins, +0.0 beats -0.0).
 #include "common.h"
 #include "kernels.h"
+#include "rowvec.h"
 #include <algorithm>
 
 namespace shk {
@@ -249,27 +250,36 @@ __global__ void __launch_bounds__(256) colsum_pass1(const float* __restrict__ x,
   if (w == 0 && col < N)
     part[(int64_t)blockIdx.y * N + col] = ((lds[0][lane] + lds[1][lane]) + lds[2][lane]) + lds[3][lane];
 }
-// Pass 1 for 16-byte-aligned rows (N and ldx multiples of 4, x 16-byte aligned): each lane owns
-// four adjacent columns and reads them with one streaming 16-byte load per row, so a wave moves
-// 1 KiB per row and a block covers 256 columns. Panels, row assignment (rows r0 + w, r0 + w + 4,
-// ...) and the combination order are those of colsum_pass1, so both write identical partials.
-__global__ void __launch_bounds__(256) colsum_pass1_v4(const float* __restrict__ x, double* part,
-                                                      int64_t R, int64_t N, int64_t ldx,
-                                                      int64_t rows) {
-  __shared__ double lds[4][4 * CS_COLS];
+// Pass 1 for wider inputs: each lane owns four adjacent columns and reads them with one streaming
+// 16-byte load per row (at any float), so a wave moves 1 KiB per row and a block covers 256
+// columns with 16 waves (rows r0 + w, r0 + w + 16, ..., four loads in flight each; a quarter of
+// colsum_pass1's blocks, so four times its waves). With 4-byte loads too few bytes are in flight:
+// [20000, 1001] 40.8 us on MI355X, 21.7 so.
+constexpr int CS_WAVES = 16;
+__global__ void __launch_bounds__(64 * CS_WAVES) colsum_pass1_v4(const float* __restrict__ x,
+                                                                double* part, int64_t R, int64_t N,
+                                                                int64_t ldx, int64_t rows) {
+  __shared__ double lds[CS_WAVES][4 * CS_COLS];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t col = ((int64_t)blockIdx.x * CS_COLS + lane) * 4;
   const int64_t r0 = (int64_t)blockIdx.y * rows;
+  const int64_t rend = min<int64_t>(R, r0 + rows);
   double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  if (col < N) {
-    const int64_t rend = min<int64_t>(R, r0 + rows);
+  if (col + 3 < N) {
 #pragma unroll 4
-    for (int64_t r = r0 + w; r < rend; r += 4) {
-      const float4 v = ld_stream(reinterpret_cast<const float4*>(x + r * ldx + col));
-      s0 += (double)v.x;
-      s1 += (double)v.y;
-      s2 += (double)v.z;
-      s3 += (double)v.w;
+    for (int64_t r = r0 + w; r < rend; r += CS_WAVES) {
+      const float4u v = __builtin_nontemporal_load(reinterpret_cast<const float4u*>(x + r * ldx + col));
+      s0 += (double)v[0];
+      s1 += (double)v[1];
+      s2 += (double)v[2];
+      s3 += (double)v[3];
+    }
+  } else if (col < N) {  // the last one to three columns
+    for (int64_t r = r0 + w; r < rend; r += CS_WAVES) {
+      const float* src = x + r * ldx + col;
+      s0 += (double)src[0];
+      if (col + 1 < N) s1 += (double)src[1];
+      if (col + 2 < N) s2 += (double)src[2];
     }
   }
   lds[w][4 * lane + 0] = s0;
@@ -279,8 +289,12 @@ __global__ void __launch_bounds__(256) colsum_pass1_v4(const float* __restrict__
   __syncthreads();
   const int c = threadIdx.x;  // one column of the block's 256 per thread
   const int64_t gc = (int64_t)blockIdx.x * 4 * CS_COLS + c;
-  if (gc < N)
-    part[(int64_t)blockIdx.y * N + gc] = ((lds[0][c] + lds[1][c]) + lds[2][c]) + lds[3][c];
+  if (c < 4 * CS_COLS && gc < N) {
+    double s = lds[0][c];
+#pragma unroll
+    for (int i = 1; i < CS_WAVES; ++i) s += lds[i][c];
+    part[(int64_t)blockIdx.y * N + gc] = s;
+  }
 }
 // Column sums of a narrow input in one launch (N <= CS_SMALL_MAX_N, R <= CS_SMALL_MAX_R): block
 // x sums 64 columns over all R rows with 16 waves (wave w: rows w, w + 16, ..., eight loads in
@@ -344,39 +358,192 @@ __global__ void __launch_bounds__(256) colsum_pass2(const double* part, float* o
   }
 }
 
-// Row reductions: one workgroup per row, binary64 accumulation for SUM/MEAN/LSE.
-template <int NT>
-__global__ void __launch_bounds__(NT) row_reduce_kernel(const float* __restrict__ x, float* out,
-                                                        int64_t C, int kind) {
-  __shared__ double dl[NT / 64];
-  __shared__ float fl[NT / 64];
-  const float* row = x + (int64_t)blockIdx.x * C;
-  if (kind == 2 || kind == 3) {
-    float m = -INFINITY;
-    for (int64_t c = threadIdx.x; c < C; c += NT) m = java_max(m, row[c]);
-    m = block_max<NT>(m, fl);
-    if (kind == 2) {
-      if (threadIdx.x == 0) out[blockIdx.x] = C == 0 ? -INFINITY : m;
-      return;
+// Row reductions, binary64 accumulation for SUM/MEAN/LSE, one read of each row in aligned 16-byte
+// groups (rowvec.h), V of them a thread held in registers (LOG_SUM_EXP looks at them twice). Rows of
+// at most 2044 take one wave each: a workgroup a row spends its time in barriers and a single
+// load's latency. Wider rows take a workgroup of 256, rows beyond 8188 are read 4 bytes at a time
+// (twice for LOG_SUM_EXP). [20000, 1001] on MI355X, one workgroup a row with 4-byte loads before:
+// MAX 39, MEAN 22, LOG_SUM_EXP 58 us; now 14, 16 and 30.
+constexpr int RR_NT = 256;
+
+__device__ __forceinline__ float row_lse(float m, float shift, double s) {
+  if (m != m) return m;
+  if (m == INFINITY) return INFINITY;
+  return shift + (float)log((double)(float)s);
+}
+
+// This thread's share of the row statistics (Math.max: a NaN anywhere gives NaN, +0 beats -0).
+// The hardware maximum skips NaN and does not order zeros; a flag and, where the maximum is a
+// zero, a second look put that right.
+template <int V>
+struct RowPart {
+  float4 v[V];
+  int n;  // groups held
+  template <int STRIDE>
+  __device__ __forceinline__ void load(const RowGroups& view, const float* row, int first, float fill) {
+    n = 0;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const bool in = first + i * STRIDE < view.groups;
+      v[i] = in ? view.load(row, first + i * STRIDE, fill) : make_float4(fill, fill, fill, fill);
+      n += in;
     }
-    // LOG_SUM_EXP: shifted exponentials, one logarithm (CpuLogSumExpEmitter.java:4-9).
-    const float shift = (m == INFINITY || m == -INFINITY) ? 0.0f : m;
-    double s = 0.0;
-    for (int64_t c = threadIdx.x; c < C; c += NT) s += (double)exp_rn(row[c] - shift);
-    s = block_sum<NT>(s, dl);
-    if (threadIdx.x == 0) {
-      float r;
-      if (m != m) r = m;
-      else if (m == INFINITY) r = INFINITY;
-      else r = shift + (float)log((double)(float)s);
-      out[blockIdx.x] = r;
-    }
-    return;
   }
-  double s = 0.0;
-  for (int64_t c = threadIdx.x; c < C; c += NT) s += (double)row[c];
-  s = block_sum<NT>(s, dl);
-  if (threadIdx.x == 0) out[blockIdx.x] = kind == 1 ? (float)(s / (double)C) : (float)s;
+  __device__ __forceinline__ float maximum(int& nan) const {
+    float m = -INFINITY;
+    nan = 0;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      m = fmaxf(m, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
+      nan |= (v[i].x != v[i].x) | (v[i].y != v[i].y) | (v[i].z != v[i].z) | (v[i].w != v[i].w);
+    }
+    return m;
+  }
+  __device__ __forceinline__ int positive_zero() const {
+    int z = 0;
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      z |= (__float_as_uint(v[i].x) == 0u) | (__float_as_uint(v[i].y) == 0u) |
+           (__float_as_uint(v[i].z) == 0u) | (__float_as_uint(v[i].w) == 0u);
+    return z;
+  }
+  __device__ __forceinline__ double sum() const {
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      s0 += (double)v[i].x;
+      s1 += (double)v[i].y;
+      s2 += (double)v[i].z;
+      s3 += (double)v[i].w;
+    }
+    return (s0 + s1) + (s2 + s3);
+  }
+  // (padding is -inf, whose exponential is 0)
+  __device__ __forceinline__ double sum_exp(float shift) const {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+      if (i < n)
+        s += ((double)exp_rn(v[i].x - shift) + (double)exp_rn(v[i].y - shift)) +
+             ((double)exp_rn(v[i].z - shift) + (double)exp_rn(v[i].w - shift));
+    return s;
+  }
+};
+
+__device__ __forceinline__ float wave_fmax(float m) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  return m;
+}
+
+// One wave a row, four rows a workgroup.
+template <int KIND, int V>
+__global__ void __launch_bounds__(RR_NT) row_reduce_wave(const float* __restrict__ x, float* out,
+                                                         int64_t R, int64_t C) {
+  const int lane = threadIdx.x & 63;
+  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (r >= R) return;
+  const float* row = x + r * C;
+  const RowGroups view(row, (int)C);
+  RowPart<V> part;
+  part.template load<64>(view, row, lane, KIND >= 2 ? -INFINITY : 0.0f);
+  float result;
+  if constexpr (KIND < 2) {
+    const double s = wave_sum(part.sum());
+    result = KIND == 1 ? (float)(s / (double)C) : (float)s;
+  } else {
+    int nan;
+    float m = wave_fmax(part.maximum(nan));
+    if (__any(nan)) m = NAN;
+    else if (m == 0.0f) m = __any(part.positive_zero()) ? 0.0f : -0.0f;
+    result = m;
+    if constexpr (KIND == 3) {
+      // LOG_SUM_EXP: shifted exponentials, one logarithm (CpuLogSumExpEmitter.java:4-9)
+      const float shift = (m == INFINITY || m == -INFINITY) ? 0.0f : m;
+      result = row_lse(m, shift, wave_sum(part.sum_exp(shift)));
+    }
+  }
+  if (lane == 0) out[r] = result;
+}
+
+// One workgroup a row; V = 0: any width.
+template <int KIND, int V>
+__global__ void __launch_bounds__(RR_NT) row_reduce_block(const float* __restrict__ x, float* out,
+                                                          int64_t R, int64_t C) {
+  __shared__ double dl[RR_NT / 64];
+  __shared__ float fl[RR_NT / 64];
+  __shared__ int nl[RR_NT / 64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  for (int64_t r = blockIdx.x; r < R; r += gridDim.x) {
+    const float* row = x + r * C;
+    __syncthreads();  // the shared values of the row before have been read
+    if constexpr (V == 0) {
+      if constexpr (KIND < 2) {
+        double s = 0.0;
+#pragma unroll 8
+        for (int64_t c = tid; c < C; c += RR_NT) s += (double)row[c];
+        s = block_sum<RR_NT>(s, dl);
+        if (tid == 0) out[r] = KIND == 1 ? (float)(s / (double)C) : (float)s;
+      } else {
+        float m = -INFINITY;
+        for (int64_t c = tid; c < C; c += RR_NT) m = java_max(m, row[c]);
+        m = block_max<RR_NT>(m, fl);
+        if constexpr (KIND == 2) {
+          if (tid == 0) out[r] = m;
+        } else {
+          const float shift = (m == INFINITY || m == -INFINITY) ? 0.0f : m;
+          double s = 0.0;
+          for (int64_t c = tid; c < C; c += RR_NT) s += (double)exp_rn(row[c] - shift);
+          s = block_sum<RR_NT>(s, dl);
+          if (tid == 0) out[r] = row_lse(m, shift, s);
+        }
+      }
+    } else {
+      const RowGroups view(row, (int)C);
+      RowPart<V> part;
+      part.template load<RR_NT>(view, row, tid, KIND >= 2 ? -INFINITY : 0.0f);
+      if constexpr (KIND < 2) {
+        const double s = block_sum<RR_NT>(part.sum(), dl);
+        if (tid == 0) out[r] = KIND == 1 ? (float)(s / (double)C) : (float)s;
+      } else {
+        int nan;
+        float m = wave_fmax(part.maximum(nan));
+        nan = __any(nan);
+        if (lane == 0) { fl[w] = m; nl[w] = nan; }
+        __syncthreads();
+        m = fmaxf(fmaxf(fl[0], fl[1]), fmaxf(fl[2], fl[3]));
+        if (nl[0] | nl[1] | nl[2] | nl[3]) {
+          m = NAN;
+        } else if (m == 0.0f) {  // the same for the whole workgroup
+          const int z = __any(part.positive_zero());
+          __syncthreads();
+          if (lane == 0) nl[w] = z;
+          __syncthreads();
+          m = (nl[0] | nl[1] | nl[2] | nl[3]) ? 0.0f : -0.0f;
+        }
+        if constexpr (KIND == 2) {
+          if (tid == 0) out[r] = m;
+        } else {
+          const float shift = (m == INFINITY || m == -INFINITY) ? 0.0f : m;
+          const double s = block_sum<RR_NT>(part.sum_exp(shift), dl);
+          if (tid == 0) out[r] = row_lse(m, shift, s);
+        }
+      }
+    }
+  }
+}
+
+template <int KIND>
+void launch_row_kind(const float* x, float* out, int64_t R, int64_t C, hipStream_t s) {
+  const dim3 rows((unsigned)std::min<int64_t>(R, 1 << 20)), quads((unsigned)((R + 3) / 4)), nt(RR_NT);
+  // V groups hold rows of at most 4 V (threads) - 4 floats: a ragged start takes up to three
+  if (C <= 64 * 4 * 1 - 4) hipLaunchKernelGGL((row_reduce_wave<KIND, 1>), quads, nt, 0, s, x, out, R, C);
+  else if (C <= 64 * 4 * 2 - 4) hipLaunchKernelGGL((row_reduce_wave<KIND, 2>), quads, nt, 0, s, x, out, R, C);
+  else if (C <= 64 * 4 * 4 - 4) hipLaunchKernelGGL((row_reduce_wave<KIND, 4>), quads, nt, 0, s, x, out, R, C);
+  else if (C <= 64 * 4 * 8 - 4) hipLaunchKernelGGL((row_reduce_wave<KIND, 8>), quads, nt, 0, s, x, out, R, C);
+  else if (C <= RR_NT * 4 * 4 - 4) hipLaunchKernelGGL((row_reduce_block<KIND, 4>), rows, nt, 0, s, x, out, R, C);
+  else if (C <= RR_NT * 4 * 8 - 4) hipLaunchKernelGGL((row_reduce_block<KIND, 8>), rows, nt, 0, s, x, out, R, C);
+  else hipLaunchKernelGGL((row_reduce_block<KIND, 0>), rows, nt, 0, s, x, out, R, C);
 }
 
 // Whole-tensor reductions in two deterministic passes.
@@ -393,9 +560,20 @@ __global__ void __launch_bounds__(256) reduce_all_pass1(const float* __restrict_
     if (threadIdx.x == 0) part[blockIdx.x] = (double)m;
     return;
   }
-  double s = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) s += (double)x[i];
-  s = block_sum<256>(s, dl);
+  // 16-byte loads, four a thread in flight ([20020000] SUM 24.4 us with 4-byte loads on MI355X,
+  // 14.4 so)
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  const int64_t n4 = n / 4;
+#pragma unroll 4
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += stride) {
+    const float4u v = __builtin_nontemporal_load(reinterpret_cast<const float4u*>(x) + i);
+    s0 += (double)v[0];
+    s1 += (double)v[1];
+    s2 += (double)v[2];
+    s3 += (double)v[3];
+  }
+  if (blockIdx.x == 0 && threadIdx.x < n - 4 * n4) s0 += (double)x[4 * n4 + threadIdx.x];
+  const double s = block_sum<256>((s0 + s1) + (s2 + s3), dl);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 __global__ void __launch_bounds__(256) reduce_all_pass2(const double* part, int P, int64_t n,
@@ -575,9 +753,9 @@ hipError_t launch_colsum(const float* x, float* out, int64_t R, int64_t N, int64
   const int64_t rows = colsum_rows_per_panel(R, N);
   const int64_t P = (R + rows - 1) / rows;
   if (P > 0) {
-    if (N % 4 == 0 && ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+    if (N >= 4 * CS_COLS) {
       dim3 g1((unsigned)((N + 4 * CS_COLS - 1) / (4 * CS_COLS)), (unsigned)P);
-      hipLaunchKernelGGL(colsum_pass1_v4, g1, dim3(256), 0, s, x, partial, R, N, ldx, rows);
+      hipLaunchKernelGGL(colsum_pass1_v4, g1, dim3(64 * CS_WAVES), 0, s, x, partial, R, N, ldx, rows);
     } else {
       dim3 g1((unsigned)((N + CS_COLS - 1) / CS_COLS), (unsigned)P);
       hipLaunchKernelGGL(colsum_pass1, g1, dim3(256), 0, s, x, partial, R, N, ldx, rows);
@@ -599,7 +777,12 @@ hipError_t launch_colsum_finish(const double* partial, float* out, int64_t P, in
 hipError_t launch_row_reduce(const float* x, float* out, int64_t R, int64_t C, int kind,
                              hipStream_t s) {
   if (R <= 0) return hipSuccess;
-  hipLaunchKernelGGL(row_reduce_kernel<256>, dim3((unsigned)R), dim3(256), 0, s, x, out, C, kind);
+  switch (kind) {
+    case 0: launch_row_kind<0>(x, out, R, C, s); break;
+    case 1: launch_row_kind<1>(x, out, R, C, s); break;
+    case 2: launch_row_kind<2>(x, out, R, C, s); break;
+    default: launch_row_kind<3>(x, out, R, C, s); break;
+  }
   return hipGetLastError();
 }
 
