@@ -67,9 +67,13 @@ struct DirectOperand {
         f[b] = floatx4{v[0], v[1], v[2], v[3]};
       }
     } else {
+      // the step's offset is opaque, or the compiler keeps a pointer of its own for every load of
+      // the unrolled steps (some 60 registers, and spills)
+      int64_t step = k * ld;
+      asm volatile("" : "+s"(step));
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const float* src = p[0] + (k + s) * ld;
+        const float* src = p[0] + step + s * ld;
         if (!edge) {
           if constexpr (NB == 4) {
             const float4u v = *reinterpret_cast<const float4u*>(src + row0);
@@ -150,7 +154,8 @@ gemm_direct(GemmParams p) {
       acc[decltype(i)::value][decltype(j)::value] = floatx4{0.f, 0.f, 0.f, 0.f};
     });
   });
-  auto mfma_step = [&](const floatx4 (&fa)[NB], const floatx4 (&fb)[NB]) {
+  auto mfma_step = [&](const floatx4 (&fa)[NB], const floatx4 (&fb)[NB])
+      __attribute__((always_inline)) {
     static_for<4>([&](auto sc) {
       constexpr int S = decltype(sc)::value;
       static_for<NB * NB>([&](auto n) {
@@ -171,7 +176,7 @@ gemm_direct(GemmParams p) {
     A.init(p.A, p.lda, rm, p.M);
     B.init(p.B, p.ldb, rn, p.N);
     floatx4 fa[D][NB], fb[D][NB];
-    static_for<D>([&](auto jc) {
+    static_for<D>([&](auto jc) __attribute__((always_inline)) {
       constexpr int J = decltype(jc)::value;
       if (J < nfull) {
         A.load(fa[J], kb + J * DK);
@@ -180,7 +185,7 @@ gemm_direct(GemmParams p) {
     });
     int t = 0;
     for (; t + 2 * D <= nfull; t += D) {
-      static_for<D>([&](auto jc) {
+      static_for<D>([&](auto jc) __attribute__((always_inline)) {
         constexpr int J = decltype(jc)::value;
         mfma_step(fa[J], fb[J]);
         __builtin_amdgcn_sched_barrier(0);
@@ -190,7 +195,7 @@ gemm_direct(GemmParams p) {
       });
     }
     // fewer than 2 D steps left, D of them in flight
-    static_for<2 * D - 1>([&](auto jc) {
+    static_for<2 * D - 1>([&](auto jc) __attribute__((always_inline)) {
       constexpr int J = decltype(jc)::value;
       if (t + J < nfull) {
         mfma_step(fa[J % D], fb[J % D]);
