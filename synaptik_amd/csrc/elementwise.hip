@@ -17,6 +17,7 @@
 #include "kernels.h"
 #include "rowvec.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace shk {
 namespace {
@@ -39,11 +40,9 @@ enum PwOp : uint8_t {
 };
 constexpr int PW_REGS = 8;
 
-// Binary64-evaluated transcendentals kept out of line: they are rare in chains, and inlining
-// them into every interpreter case inflates the register allocation of the whole kernel.
-__device__ __noinline__ float pw_tanh(float a) { return tanh_f(a); }
-__device__ __noinline__ float pw_sigmoid(float a) { return sigmoid_f(a); }
-__device__ __noinline__ float pw_exp(float a) { return exp_rn(a); }
+// Library functions kept out of line: they are rare in chains, and inlining them into the
+// interpreter inflates the register allocation of the whole kernel. (exp, tanh and sigmoid are
+// short: fexp64.h.)
 __device__ __noinline__ float pw_log(float a) { return (float)log((double)a); }
 __device__ __noinline__ float pw_sqrt(float a) { return (float)sqrt((double)a); }
 
@@ -58,9 +57,9 @@ __device__ __forceinline__ float pw_op(int op, float a, float b, float c, float 
     case PW_DIV: return a / b;
     case PW_NEG: return -a;
     case PW_RELU: return relu_f(a);
-    case PW_TANH: return pw_tanh(a);
-    case PW_SIGMOID: return pw_sigmoid(a);
-    case PW_EXP: return pw_exp(a);
+    case PW_TANH: return tanh_f(a);
+    case PW_SIGMOID: return sigmoid_f(a);
+    case PW_EXP: return exp_rn(a);
     case PW_LOG: return pw_log(a);
     case PW_RELU_GRAD: return act_grad(ACT_RELU, b, a);
     case PW_TANH_GRAD: return act_grad(ACT_TANH, b, a);
@@ -72,6 +71,12 @@ __device__ __forceinline__ float pw_op(int op, float a, float b, float c, float 
     case PW_SQRT: return pw_sqrt(a);
     default: return 0.0f;
   }
+}
+
+constexpr bool pw_reads_b(int op) {
+  return op == PW_ADD || op == PW_SUB || op == PW_MUL || op == PW_DIV || op == PW_MAX ||
+         op == PW_GT || op == PW_RELU_GRAD || op == PW_TANH_GRAD || op == PW_SIGMOID_GRAD ||
+         op == PW_WHERE;
 }
 
 // Single-op chains (LOAD x [, LOAD y], OP, STORE) over full-shape, 16-byte aligned operands (out
@@ -107,92 +112,172 @@ __global__ void __launch_bounds__(256) pw_single_kernel(const float* x,
   }
 }
 
-// Loads input k for the 4-element group starting at e0 (cnt valid elements) into v.
-__device__ __forceinline__ void pw_load4(const PwParams& p, int k, int64_t e0, int cnt, float (&v)[4]) {
-  const float* src = p.in[k];
-  switch (p.in_mode[k]) {
-    case 0:
-      if (cnt == 4 && (reinterpret_cast<uintptr_t>(src + e0) & 15u) == 0) {
-        const float4 t = ld_stream(reinterpret_cast<const float4*>(src + e0));
-        v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-      } else {
-        for (int q = 0; q < cnt; ++q) v[q] = src[e0 + q];
-      }
-      break;
-    case 3: {
-      const float t = src[0];
-      v[0] = v[1] = v[2] = v[3] = t;
-      break;
-    }
-    default: {
-      // one division per group, then walk (row, col) forward
-      int64_t row = e0 / p.C, col = e0 - row * p.C;
-      for (int q = 0; q < cnt; ++q) {
-        v[q] = p.in_mode[k] == 1 ? src[col] : src[row];
-        if (++col == p.C) { col = 0; ++row; }
-      }
-    }
-  }
+// Division of element ordinals below 2^32 by the row width C (Granlund and Montgomery, "Division
+// by invariant integers using multiplication", 1994): with l = ceil(log2 C) and
+// mul = floor(2^32 (2^l - C) / C) + 1, t = high half of mul n and n / C = (t + (n - t) / 2) >> (l - 1).
+struct PwDivide {
+  uint32_t mul, shift;
+  int narrow;  // every ordinal fits 32 bits and C > 1
+};
+PwDivide pw_divide(int64_t n, int64_t C) {
+  PwDivide d{0, 0, 0};
+  if (C <= 1 || n > 0xffffffffll) return d;
+  int l = 0;
+  while ((1ll << l) < C) ++l;
+  d.mul = (uint32_t)((((unsigned __int128)1 << 32) * (uint64_t)((1ll << l) - C)) / (uint64_t)C + 1);
+  d.shift = (uint32_t)(l - 1);
+  d.narrow = 1;
+  return d;
 }
 
-// The interpreter's register file lives in LDS: register k of thread t holds its 4 elements at
-// regs[k][t*4 .. t*4+3]. Any register index is then just an address (no dynamically indexed
-// VGPR array, no scratch), and each operand access is one 128-bit LDS access per lane.
+// The interpreter. A thread handles one group of four elements, whose register k lives in LDS at
+// regs[k * PW_NT + t]: any register index is just an address (no dynamically indexed VGPR array, no
+// scratch) and each operand access is one 128-bit LDS access per lane. A launch takes only as many
+// registers as its chain uses.
+//
+// What bounds it is the instructions around the arithmetic -- decoding, branching on the operation
+// and on each input's kind -- and how many waves share them: seven a SIMD. An ordinal is divided
+// once, by multiplication; a broadcast operand within one row is one vector load; an instruction
+// is read as words (read as bytes it would come through vector memory: scalar loads have none), the
+// next one's ahead of time. Before: a 64-bit division and four loads for each broadcast operand,
+// five workgroups a CU whatever the chain. [20000, 1001] on MI355X: x - row 75 -> 44 us;
+// tanh(d / row * row + row) 176 -> 123. (Two groups a thread 56 and 153, four 107 and 180, for
+// want of registers; one group with every input loaded ahead 70 to 77 and 145 to 151.)
 constexpr int PW_NT = 256;
-struct PwRegs {
-  float4 v[PW_REGS][PW_NT];
+
+struct PwArgs {
+  PwParams p;
+  PwDivide div;
 };
 
-__device__ __forceinline__ void pw_exec(const PwParams& p, PwRegs& R, int64_t e0, int cnt,
-                                        float (&outv)[PW_MAX_OUTPUTS][4]) {
-  const int t = threadIdx.x;
-  for (int pc = 0; pc < p.n_instr; ++pc) {
-    const PwInstr ins = p.code[pc];
-    float4& d4 = R.v[ins.dst & (PW_REGS - 1)][t];
-    if (ins.op == PW_LOAD) {
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-      pw_load4(p, ins.a % PW_MAX_INPUTS, e0, cnt, v);
-      d4 = make_float4(v[0], v[1], v[2], v[3]);
-      continue;
-    }
-    const float4 a4 = R.v[ins.a & (PW_REGS - 1)][t];
-    const float4 b4 = R.v[ins.b & (PW_REGS - 1)][t];
-    const float a[4] = {a4.x, a4.y, a4.z, a4.w};
-    const float b[4] = {b4.x, b4.y, b4.z, b4.w};
-    float c[4] = {0.f, 0.f, 0.f, 0.f};
-    if (ins.op == PW_WHERE) {
-      const float4 c4 = R.v[ins.c & (PW_REGS - 1)][t];
-      c[0] = c4.x; c[1] = c4.y; c[2] = c4.z; c[3] = c4.w;
-    }
-    float d[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) d[q] = pw_op(ins.op, a[q], b[q], c[q], ins.imm);
-    if (ins.op == PW_STORE) {
-      float* o = outv[ins.dst & 1];
-      o[0] = d[0]; o[1] = d[1]; o[2] = d[2]; o[3] = d[3];
-    } else {
-      d4 = make_float4(d[0], d[1], d[2], d[3]);
-    }
-  }
+struct PwWords {
+  uint32_t w0, w1, w2;  // op | dst << 8 | a << 16 | b << 24; c; imm
+};
+static_assert(sizeof(PwInstr) == sizeof(PwWords) && alignof(PwInstr) == 4, "three words");
+__device__ __forceinline__ PwWords pw_fetch(const PwParams& p, int pc) {
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(p.code) + 3 * pc;
+  return PwWords{w[0], w[1], w[2]};
 }
 
-__global__ void __launch_bounds__(PW_NT) pointwise_kernel(PwParams p) {
-  __shared__ PwRegs regs;
+__device__ __forceinline__ float4 pw_vec(const float* src) {
+  const float4u v = *reinterpret_cast<const float4u*>(src);
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// Element by element: the group of four from e0 on, cnt of them valid, at (row, col).
+__device__ __forceinline__ float4 pw_load_each(const float* src, int mode, int64_t C, int64_t e0,
+                                               int cnt, int64_t row, int64_t col) {
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (q < cnt) {
+      v[q] = src[mode == 0 ? e0 + q : mode == 1 ? col : mode == 2 ? row : 0];
+      if (++col == C) { col = 0; ++row; }
+    }
+  }
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// BCAST: some input is a row or a column vector. WIDE: ordinals beyond 32 bits (or C == 1).
+template <bool BCAST, bool WIDE>
+__global__ void __launch_bounds__(PW_NT) __attribute__((amdgpu_waves_per_eu(7)))
+pointwise_kernel(PwArgs a) {
+  using Place = typename std::conditional<WIDE, int64_t, uint32_t>::type;
+  extern __shared__ float4 regs[];
+  const PwParams& p = a.p;
   const int64_t n = p.R * p.C;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x * 4;
-  for (int64_t e0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; e0 < n; e0 += stride) {
-    const int cnt = (int)min<int64_t>(4, n - e0);
-    float outv[PW_MAX_OUTPUTS][4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    pw_exec(p, regs, e0, cnt, outv);
-    // Stores: vectorized when the group is complete and aligned.
+  const int t = threadIdx.x;
+  const Place C = (Place)p.C;
+  constexpr int64_t TILE = (int64_t)PW_NT * 4;
+  for (int64_t base = (int64_t)blockIdx.x * TILE; base < n; base += (int64_t)gridDim.x * TILE) {
+    const bool whole = base + TILE <= n;  // uniform: every group has four elements
+    const int64_t e0 = base + t * 4;
+    auto count = [&]() { return (int)max<int64_t>(0, min<int64_t>(4, n - e0)); };
+    Place row = 0, col = 0;
+    if constexpr (BCAST) {
+      if constexpr (WIDE) {
+        row = e0 / C;
+        col = e0 - row * C;
+      } else {
+        const uint32_t e = (uint32_t)e0, h = __umulhi(a.div.mul, e);
+        row = (h + ((e - h) >> 1)) >> a.div.shift;
+        col = e - row * C;
+      }
+    }
+    // (stored after the whole chain: an output may be one of the inputs)
+    float4 outv[PW_MAX_OUTPUTS];
+    outv[0] = outv[1] = make_float4(0.f, 0.f, 0.f, 0.f);
+    PwWords next = pw_fetch(p, 0);
+    for (int pc = 0; pc < p.n_instr; ++pc) {
+      const PwWords ins = next;
+      if (pc + 1 < p.n_instr) next = pw_fetch(p, pc + 1);
+      const int op = ins.w0 & 0xff, dst = (ins.w0 >> 8) & 0xff;
+      const float imm = __uint_as_float(ins.w2);
+      float4* const D = regs + (dst & (PW_REGS - 1)) * PW_NT + t;
+      if (op == PW_LOAD) {
+        const int k = ((ins.w0 >> 16) & 0xff) % PW_MAX_INPUTS;
+        const float* src = p.in[k];
+        const int mode = (int)p.in_mode[k];
+        float4 v;
+        if (mode == 3) {
+          const float x = src[0];
+          v = make_float4(x, x, x, x);
+        } else if (mode == 0 && whole) {
+          const float4u x = __builtin_nontemporal_load(reinterpret_cast<const float4u*>(src + e0));
+          v = make_float4(x[0], x[1], x[2], x[3]);
+        } else if (!whole) {
+          v = pw_load_each(src, mode, p.C, e0, count(), row, col);
+        } else if (col + 3 >= C) {  // spans rows
+          v = pw_load_each(src, mode, p.C, e0, 4, row, col);
+        } else if (mode == 1) {
+          v = pw_vec(src + col);
+        } else {
+          const float x = src[row];
+          v = make_float4(x, x, x, x);
+        }
+        *D = v;
+        continue;
+      }
+      const float4* const A = regs + ((ins.w0 >> 16) & (PW_REGS - 1)) * PW_NT + t;
+      const float4* const B = regs + ((ins.w0 >> 24) & (PW_REGS - 1)) * PW_NT + t;
+      const float4* const Cc = regs + (ins.w1 & (PW_REGS - 1)) * PW_NT + t;
+      float4 d;
+#define PW_CASE(OP)                                                                             \
+  case OP: {                                                                                    \
+    const float4 x = *A;                                                                        \
+    const float4 y = pw_reads_b(OP) ? *B : x;                                                   \
+    const float4 z = OP == PW_WHERE ? *Cc : x;                                                  \
+    d = make_float4(pw_op(OP, x.x, y.x, z.x, imm), pw_op(OP, x.y, y.y, z.y, imm),               \
+                    pw_op(OP, x.z, y.z, z.z, imm), pw_op(OP, x.w, y.w, z.w, imm));              \
+  } break;
+      switch (op) {  // (uniform)
+        PW_CASE(PW_CONST) PW_CASE(PW_ADD) PW_CASE(PW_SUB) PW_CASE(PW_MUL) PW_CASE(PW_DIV)
+        PW_CASE(PW_NEG) PW_CASE(PW_RELU) PW_CASE(PW_TANH) PW_CASE(PW_SIGMOID) PW_CASE(PW_EXP)
+        PW_CASE(PW_LOG) PW_CASE(PW_RELU_GRAD) PW_CASE(PW_TANH_GRAD) PW_CASE(PW_SIGMOID_GRAD)
+        PW_CASE(PW_GT) PW_CASE(PW_WHERE) PW_CASE(PW_STORE) PW_CASE(PW_MAX) PW_CASE(PW_SQRT)
+        default: d = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+#undef PW_CASE
+      if (op == PW_STORE) {
+        if (dst & 1) outv[1] = d;
+        else outv[0] = d;
+      } else {
+        *D = d;
+      }
+    }
 #pragma unroll
     for (int o = 0; o < PW_MAX_OUTPUTS; ++o) {
       if (p.out[o] == nullptr) continue;
       float* dst = p.out[o] + e0;
-      if (cnt == 4 && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
-        st_stream(reinterpret_cast<float4*>(dst), make_float4(outv[o][0], outv[o][1], outv[o][2], outv[o][3]));
+      const float4 v = outv[o];
+      if (whole) {
+        __builtin_nontemporal_store(float4u{v.x, v.y, v.z, v.w}, reinterpret_cast<float4u*>(dst));
       } else {
-        for (int q = 0; q < cnt; ++q) dst[q] = outv[o][q];
+        const int cnt = count();
+        if (cnt > 0) dst[0] = v.x;
+        if (cnt > 1) dst[1] = v.y;
+        if (cnt > 2) dst[2] = v.z;
+        if (cnt > 3) dst[3] = v.w;
       }
     }
   }
@@ -697,7 +782,21 @@ hipError_t launch_pointwise(const PwParams& p, hipStream_t s) {
     case PW_LOG: launch_single<PW_LOG>(a, b, out, n, bin, s); break;
     case PW_SQRT: launch_single<PW_SQRT>(a, b, out, n, bin, s); break;
     default:
-      hipLaunchKernelGGL(pointwise_kernel, dim3(grid_for(n, 4)), dim3(PW_NT), 0, s, p);
+      PwArgs a{p, pw_divide(p.R * p.C, p.C)};
+      bool bcast = false;
+      for (int k = 0; k < PW_MAX_INPUTS; ++k)
+        bcast |= p.in[k] != nullptr && (p.in_mode[k] == 1 || p.in_mode[k] == 2);
+      int regs = 1;  // registers the chain names (every operand field is read, used or not)
+      for (int i = 0; i < p.n_instr; ++i) {
+        const PwInstr& c = p.code[i];
+        for (int r : {(int)c.dst, (int)c.a, (int)c.b, (int)c.c})
+          regs = std::max(regs, (r & (PW_REGS - 1)) + 1);
+      }
+      const size_t lds = (size_t)regs * PW_NT * sizeof(float4);
+      const dim3 g(grid_for(n, 4)), nt(PW_NT);
+      if (!bcast) hipLaunchKernelGGL((pointwise_kernel<false, false>), g, nt, lds, s, a);
+      else if (a.div.narrow) hipLaunchKernelGGL((pointwise_kernel<true, false>), g, nt, lds, s, a);
+      else hipLaunchKernelGGL((pointwise_kernel<true, true>), g, nt, lds, s, a);
   }
   return hipGetLastError();
 }
