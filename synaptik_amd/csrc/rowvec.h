@@ -22,10 +22,14 @@ struct RowGroups {
   __device__ __forceinline__ bool whole(int q) const {
     return first(q) >= 0 && first(q) + 4 <= width;
   }
-  // Group q of the row; floats outside it read as `fill`. q < groups.
+  // Group q of the row, or of another tensor's row of the same width; floats outside it read as
+  // `fill`. q < groups.
   __device__ __forceinline__ float4 load(const float* row, int q, float fill) const {
     const int c = first(q);
-    if (whole(q)) return ld_stream(reinterpret_cast<const float4*>(row + c));
+    if (whole(q)) {
+      const float4u t = __builtin_nontemporal_load(reinterpret_cast<const float4u*>(row + c));
+      return make_float4(t[0], t[1], t[2], t[3]);
+    }
     float4 v;
     v.x = c >= 0 && c < width ? row[c] : fill;
     v.y = c + 1 >= 0 && c + 1 < width ? row[c + 1] : fill;
@@ -33,8 +37,11 @@ struct RowGroups {
     v.w = c + 3 < width ? row[c + 3] : fill;
     return v;
   }
-  // Writes group q to `row`, which may be another tensor's row of the same width (it need not
-  // share the alignment of the one read).
+  // Whether float j of group q belongs to the row.
+  __device__ __forceinline__ bool holds(int q, int j) const {
+    return first(q) + j >= 0 && first(q) + j < width;
+  }
+  // Writes group q likewise. (Another tensor's row need not share the alignment of this one.)
   __device__ __forceinline__ void store(float* row, int q, const float4& v) const {
     const int c = first(q);
     if (whole(q)) {

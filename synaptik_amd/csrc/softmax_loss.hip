@@ -17,7 +17,9 @@
 #include "common.h"
 #include "fexp.h"
 #include "kernels.h"
+#include "rowvec.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace shk {
 namespace {
@@ -227,6 +229,254 @@ __global__ void __launch_bounds__(SM_NT) softmax_fwd_regs(const float* __restric
   }
 }
 
+// Rows of any start and width in aligned 16-byte groups (rowvec.h), V of them a thread, held in
+// registers from the load to the store; sums in binary64 throughout. One wave a row (NT = 64, four
+// rows a workgroup, no barrier) up to 2044 columns, where a workgroup a row spends its time in
+// barriers and a single load's latency; one workgroup of NT threads above. Aligned rows
+// of 509 to 4096 keep softmax_fwd_regs (20000x1000 97 us against 119). Three passes of 4-byte loads
+// before; us on MI355X, softmax with its gradient: 20000x1001 174 -> 103, 10000x4095 320 -> 204,
+// 2000x32000 545 -> 302, 65536x100 152 -> 84; log-softmax 92 -> 55, 157 -> 93, 271 -> 131, 122 -> 62.
+template <int NT>
+struct RowTeam {  // the threads that share a row: a wave, or a workgroup
+  static constexpr int WAVES = NT == 64 ? 4 : NT / 64;
+  static constexpr int THREADS = NT == 64 ? 256 : NT;
+  struct Shared {
+    double d[WAVES];
+    float a[WAVES], b[WAVES];
+    int i[WAVES], j[WAVES];
+  };
+  __device__ static __forceinline__ int lane() { return NT == 64 ? threadIdx.x & 63 : threadIdx.x; }
+  __device__ static __forceinline__ double sum(double v, Shared& s) {
+    v = wave_sum(v);
+    if constexpr (NT == 64) return v;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) s.d[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double r = 0.0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) r += s.d[w];
+    return r;
+  }
+  __device__ static __forceinline__ void extremes(float& mx, float& mn, Shared& s) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      mn = fminf(mn, __shfl_xor(mn, o, 64));
+    }
+    if constexpr (NT == 64) return;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) { s.a[threadIdx.x >> 6] = mx; s.b[threadIdx.x >> 6] = mn; }
+    __syncthreads();
+    mx = s.a[0];
+    mn = s.b[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) { mx = fmaxf(mx, s.a[w]); mn = fminf(mn, s.b[w]); }
+  }
+  __device__ static __forceinline__ void either(int& a, int& b, Shared& s) {
+    a = __any(a);
+    b = __any(b);
+    if constexpr (NT == 64) return;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) { s.i[threadIdx.x >> 6] = a; s.j[threadIdx.x >> 6] = b; }
+    __syncthreads();
+    a = b = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) { a |= s.i[w]; b |= s.j[w]; }
+  }
+};
+
+// exp(x - shift) with the binary64 evaluation of fexp64.h outside exp_f32's fast range.
+__device__ __forceinline__ float row_exp(float x, float shift) {
+  const float t = x - shift;
+  return t >= -87.0f && t <= 88.0f ? exp_f32_in_range(t) : exp_rn(t);
+}
+
+template <int NT, int V, bool LOG>
+__global__ void __launch_bounds__(RowTeam<NT>::THREADS)
+__attribute__((amdgpu_waves_per_eu(NT == 1024 ? 4 : V <= 2 ? 5 : V == 4 ? 4 : 3)))
+softmax_fwd_rows(const float* x, float* y, float* lse, int64_t R, int64_t C) {
+  using Team = RowTeam<NT>;
+  __shared__ typename Team::Shared sh;
+  const int tid = Team::lane();
+  const int64_t first_row = NT == 64 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  const int64_t row_step = NT == 64 ? (int64_t)gridDim.x * 4 : gridDim.x;
+  for (int64_t r = first_row; r < R; r += row_step) {
+    const float* xr = x + r * C;
+    float* yr = y + r * C;
+    const RowGroups view(xr, (int)C);
+    float4 v[V];
+    float m = -INFINITY, mn = INFINITY;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int q = tid + i * NT;
+      v[i] = q < view.groups ? view.load(xr, q, -INFINITY)
+                             : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int q = tid + i * NT;
+      m = fmaxf(m, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
+      if (q < view.groups) {
+        if (view.whole(q)) {
+          mn = fminf(mn, fminf(fminf(v[i].x, v[i].y), fminf(v[i].z, v[i].w)));
+        } else {
+          if (view.holds(q, 0)) mn = fminf(mn, v[i].x);
+          if (view.holds(q, 1)) mn = fminf(mn, v[i].y);
+          if (view.holds(q, 2)) mn = fminf(mn, v[i].z);
+          if (view.holds(q, 3)) mn = fminf(mn, v[i].w);
+        }
+      }
+    }
+    Team::extremes(m, mn, sh);
+    if (m == INFINITY || m == 0.0f) {  // uniform for the row, rare (see softmax_fwd_regs)
+      int nan = 0, pos_zero = 0;
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        nan |= (v[i].x != v[i].x) | (v[i].y != v[i].y) | (v[i].z != v[i].z) | (v[i].w != v[i].w);
+        pos_zero |= (__float_as_uint(v[i].x) == 0u) | (__float_as_uint(v[i].y) == 0u) |
+                    (__float_as_uint(v[i].z) == 0u) | (__float_as_uint(v[i].w) == 0u);
+      }
+      Team::either(nan, pos_zero, sh);
+      if (nan) m = NAN;
+      else if (m == 0.0f) m = pos_zero ? 0.0f : -0.0f;
+    }
+    if (m == INFINITY) {
+      const float other = LOG ? -INFINITY : 0.0f;
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        const int q = tid + i * NT;
+        if (q < view.groups)
+          view.store(yr, q, make_float4(v[i].x == INFINITY ? NAN : other, v[i].y == INFINITY ? NAN : other,
+                                        v[i].z == INFINITY ? NAN : other, v[i].w == INFINITY ? NAN : other));
+      }
+      if (lse != nullptr && tid == 0) lse[r] = INFINITY;
+      continue;
+    }
+    const bool neg_inf = mn == -INFINITY;
+    const float shift = (neg_inf && m == m) ? 0.0f : m;
+    // every argument in the binary32 exponential's range (see softmax_fwd_regs)
+    const bool in_range = shift == m && is_finite(m) && mn - m >= -87.0f;
+    // (padding, -inf, lies outside that range: its terms are left out)
+    auto add = [&](int i, const float4& e, double& s) {
+      const int q = tid + i * NT;
+      if (q >= view.groups) return;
+      if (view.whole(q)) {
+        s += ((double)e.x + (double)e.y) + ((double)e.z + (double)e.w);
+      } else {
+        if (view.holds(q, 0)) s += (double)e.x;
+        if (view.holds(q, 1)) s += (double)e.y;
+        if (view.holds(q, 2)) s += (double)e.z;
+        if (view.holds(q, 3)) s += (double)e.w;
+      }
+    };
+    float row_lse = 0.0f;
+    const bool lse_apart = lse != nullptr && neg_inf && is_finite(m);
+    if (lse_apart) {
+      // LOG_SUM_EXP keeps the maximum as its shift even when the row holds -inf
+      // (CpuLogSumExpEmitter.java:4-9); only the softmax values use the unshifted form.
+      double s2 = 0.0;
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        add(i, make_float4(row_exp(v[i].x, m), row_exp(v[i].y, m), row_exp(v[i].z, m),
+                           row_exp(v[i].w, m)), s2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      row_lse = m + (float)log((double)(float)Team::sum(s2, sh));
+    }
+    double s = 0.0;
+    auto exps = [&](auto fast) {
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        float4 e;
+        if constexpr (decltype(fast)::value) {
+          e = make_float4(exp_f32_in_range(v[i].x - shift), exp_f32_in_range(v[i].y - shift),
+                          exp_f32_in_range(v[i].z - shift), exp_f32_in_range(v[i].w - shift));
+        } else {
+          e = make_float4(row_exp(v[i].x, shift), row_exp(v[i].y, shift),
+                          row_exp(v[i].z, shift), row_exp(v[i].w, shift));
+        }
+        add(i, e, s);
+        if constexpr (!LOG) v[i] = e;
+        __builtin_amdgcn_sched_barrier(0);  // four at a time keep the registers down
+      }
+    };
+    if (in_range) exps(std::true_type{});
+    else exps(std::false_type{});
+    const float sum = (float)Team::sum(s, sh);
+    // softmax needs the logarithm of the sum for the LSE output alone
+    const float logsum = LOG || tid == 0 ? (float)log((double)sum) : 0.0f;
+    // In range the sum lies in [1, C], and a reciprocal with a residual correction gives the
+    // correctly rounded quotient; otherwise divide.
+    const float inv = 1.0f / sum;
+    auto quotient = [&](float e) {
+      if (!in_range) return e / sum;
+      const float q0 = e * inv;
+      return fmaf(fmaf(-q0, sum, e), inv, q0);
+    };
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int q = tid + i * NT;
+      if (q < view.groups) {
+        float4 o;
+        if constexpr (LOG)
+          o = make_float4((v[i].x - shift) - logsum, (v[i].y - shift) - logsum,
+                          (v[i].z - shift) - logsum, (v[i].w - shift) - logsum);
+        else
+          o = make_float4(quotient(v[i].x), quotient(v[i].y), quotient(v[i].z), quotient(v[i].w));
+        view.store(yr, q, o);
+      }
+    }
+    if (lse != nullptr && tid == 0) lse[r] = lse_apart ? row_lse : shift + logsum;
+  }
+}
+
+// dX = y (.) (g - s) [+ k_r * y], s = sum(g (.) y), over the same row forms.
+template <int NT, int V>
+__global__ void __launch_bounds__(RowTeam<NT>::THREADS)
+softmax_bwd_rows(const float* y, const float* g, float* dx, int64_t R, int64_t C,
+                 const float* rowscale, float rsc) {
+  using Team = RowTeam<NT>;
+  __shared__ typename Team::Shared sh;
+  const int tid = Team::lane();
+  const int64_t first_row = NT == 64 ? (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+  const int64_t row_step = NT == 64 ? (int64_t)gridDim.x * 4 : gridDim.x;
+  const bool scaled = rowscale != nullptr || rsc != 0.0f;
+  for (int64_t r = first_row; r < R; r += row_step) {
+    const float* yr = y + r * C;
+    const float* gr = g + r * C;
+    const RowGroups view(yr, (int)C);
+    float4 yv[V], gv[V];
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int q = tid + i * NT;
+      yv[i] = q < view.groups ? view.load(yr, q, 0.0f) : zero;
+      gv[i] = q < view.groups ? view.load(gr, q, 0.0f) : zero;
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      s += (double)(gv[i].x * yv[i].x);
+      s += (double)(gv[i].y * yv[i].y);
+      s += (double)(gv[i].z * yv[i].z);
+      s += (double)(gv[i].w * yv[i].w);
+    }
+    const float sf = (float)Team::sum(s, sh);
+    const float k = rowscale != nullptr ? rowscale[r] : rsc;
+    auto out = [&](float a, float b) {
+      const float o = a * (b - sf);
+      return scaled ? o + k * a : o;
+    };
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const int q = tid + i * NT;
+      if (q < view.groups)
+        view.store(dx + r * C, q, make_float4(out(yv[i].x, gv[i].x), out(yv[i].y, gv[i].y),
+                                              out(yv[i].z, gv[i].z), out(yv[i].w, gv[i].w)));
+    }
+  }
+}
+
 // Any width: three streaming passes over the row.
 __global__ void __launch_bounds__(SM_NT) softmax_fwd_stream(const float* __restrict__ x,
                                                             float* __restrict__ y, float* lse,
@@ -415,19 +665,55 @@ __global__ void __launch_bounds__(256) mse_pass2(const double* part, int P, int6
 
 }  // namespace
 
+namespace {
+// One wave a row: four rows a workgroup; otherwise a row a workgroup (looping beyond 2^20).
+template <int NT>
+dim3 row_grid(int64_t R) {
+  return dim3((unsigned)std::min<int64_t>(NT == 64 ? (R + 3) / 4 : R, 1 << 20));
+}
+template <int NT, int V>
+void launch_fwd_rows(const float* x, float* y, float* lse, int64_t R, int64_t C, int log_softmax,
+                     hipStream_t s) {
+  const dim3 g = row_grid<NT>(R), b(RowTeam<NT>::THREADS);
+  if (log_softmax) hipLaunchKernelGGL((softmax_fwd_rows<NT, V, true>), g, b, 0, s, x, y, lse, R, C);
+  else hipLaunchKernelGGL((softmax_fwd_rows<NT, V, false>), g, b, 0, s, x, y, lse, R, C);
+}
+template <int NT, int V>
+void launch_bwd_rows(const float* y, const float* g, float* dx, int64_t R, int64_t C,
+                     const float* rowscale, float rsc, hipStream_t s) {
+  hipLaunchKernelGGL((softmax_bwd_rows<NT, V>), row_grid<NT>(R), dim3(RowTeam<NT>::THREADS), 0, s,
+                     y, g, dx, R, C, rowscale, rsc);
+}
+// Floats that V groups of each of NT threads hold, whatever the row's start.
+constexpr int64_t row_capacity(int nt, int v) { return 4ll * nt * v - 4; }
+}  // namespace
+
 hipError_t launch_softmax_fwd(const float* x, float* y, float* lse, int64_t R, int64_t C,
                               int log_softmax, hipStream_t s) {
   if (R <= 0) return hipSuccess;
   const bool vec = C % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0;
-  dim3 g((unsigned)R), b(SM_NT);
-  if (vec && C > 0 && C <= 1024)
-    hipLaunchKernelGGL(softmax_fwd_regs<1>, g, b, 0, s, x, y, lse, C, log_softmax);
-  else if (vec && C > 0 && C <= 2048)
-    hipLaunchKernelGGL(softmax_fwd_regs<2>, g, b, 0, s, x, y, lse, C, log_softmax);
-  else if (vec && C > 0 && C <= 4096)
-    hipLaunchKernelGGL(softmax_fwd_regs<4>, g, b, 0, s, x, y, lse, C, log_softmax);
+  auto rows = [&](auto nt, auto v) {
+    launch_fwd_rows<decltype(nt)::value, decltype(v)::value>(x, y, lse, R, C, log_softmax, s);
+  };
+  auto regs = [&](auto v) {
+    hipLaunchKernelGGL(softmax_fwd_regs<decltype(v)::value>, dim3((unsigned)R), dim3(SM_NT), 0, s, x, y, lse, C, log_softmax);
+  };
+  using std::integral_constant;
+  if (C <= 0)
+    hipLaunchKernelGGL(softmax_fwd_stream, dim3((unsigned)R), dim3(SM_NT), 0, s, x, y, lse, C, log_softmax);
+  else if (C <= row_capacity(64, 1)) rows(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+  else if (C <= row_capacity(64, 2)) rows(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+  else if (vec && C <= 1024) regs(integral_constant<int, 1>{});
+  else if (vec && C <= 2048) regs(integral_constant<int, 2>{});
+  else if (vec && C <= 4096) regs(integral_constant<int, 4>{});
+  else if (C <= row_capacity(64, 4)) rows(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+  else if (C <= row_capacity(64, 8)) rows(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+  else if (C <= row_capacity(256, 4)) rows(integral_constant<int, 256>{}, integral_constant<int, 4>{});
+  else if (C <= row_capacity(256, 8)) rows(integral_constant<int, 256>{}, integral_constant<int, 8>{});
+  else if (C <= row_capacity(512, 8)) rows(integral_constant<int, 512>{}, integral_constant<int, 8>{});
+  else if (C <= row_capacity(1024, 8) + (vec ? 4 : 0)) rows(integral_constant<int, 1024>{}, integral_constant<int, 8>{});
   else
-    hipLaunchKernelGGL(softmax_fwd_stream, g, b, 0, s, x, y, lse, C, log_softmax);
+    hipLaunchKernelGGL(softmax_fwd_stream, dim3((unsigned)R), dim3(SM_NT), 0, s, x, y, lse, C, log_softmax);
   return hipGetLastError();
 }
 
@@ -437,15 +723,29 @@ hipError_t launch_softmax_bwd(const float* y, const float* g, float* dx, int64_t
   const bool vec = C % 4 == 0 &&
       ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(g) |
         reinterpret_cast<uintptr_t>(dx)) & 15u) == 0;
-  dim3 gr((unsigned)R), b(SM_NT);
-  if (vec && C > 0 && C <= 1024)
-    hipLaunchKernelGGL(softmax_bwd_regs<1>, gr, b, 0, s, y, g, dx, C, rowscale, rowscale_const);
-  else if (vec && C > 0 && C <= 2048)
-    hipLaunchKernelGGL(softmax_bwd_regs<2>, gr, b, 0, s, y, g, dx, C, rowscale, rowscale_const);
-  else if (vec && C > 0 && C <= 4096)
-    hipLaunchKernelGGL(softmax_bwd_regs<4>, gr, b, 0, s, y, g, dx, C, rowscale, rowscale_const);
+  auto rows = [&](auto nt, auto v) {
+    launch_bwd_rows<decltype(nt)::value, decltype(v)::value>(y, g, dx, R, C, rowscale, rowscale_const, s);
+  };
+  auto regs = [&](auto v) {
+    hipLaunchKernelGGL(softmax_bwd_regs<decltype(v)::value>, dim3((unsigned)R), dim3(SM_NT), 0, s, y, g, dx, C, rowscale,
+                       rowscale_const);
+  };
+  using std::integral_constant;
+  if (C <= 0) return hipSuccess;
+  if (C <= row_capacity(64, 1)) rows(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+  else if (C <= row_capacity(64, 2)) rows(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+  else if (vec && C <= 1024) regs(integral_constant<int, 1>{});
+  else if (vec && C <= 2048) regs(integral_constant<int, 2>{});
+  else if (vec && C <= 4096) regs(integral_constant<int, 4>{});
+  else if (C <= row_capacity(64, 4)) rows(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+  else if (C <= row_capacity(64, 8)) rows(integral_constant<int, 64>{}, integral_constant<int, 8>{});
+  else if (C <= row_capacity(256, 4)) rows(integral_constant<int, 256>{}, integral_constant<int, 4>{});
+  else if (C <= row_capacity(256, 8)) rows(integral_constant<int, 256>{}, integral_constant<int, 8>{});
+  else if (C <= row_capacity(512, 8)) rows(integral_constant<int, 512>{}, integral_constant<int, 8>{});
+  else if (C <= row_capacity(1024, 8) + (vec ? 4 : 0)) rows(integral_constant<int, 1024>{}, integral_constant<int, 8>{});
   else
-    hipLaunchKernelGGL(softmax_bwd_stream, gr, b, 0, s, y, g, dx, C, rowscale, rowscale_const);
+    hipLaunchKernelGGL(softmax_bwd_stream, dim3((unsigned)R), dim3(SM_NT), 0, s, y, g, dx, C, rowscale,
+                       rowscale_const);
   return hipGetLastError();
 }
 

@@ -1,0 +1,82 @@
+"""Softmax, log-softmax, log-sum-exp and the softmax gradient at the edges of their row forms (one
+wave a row up to 2044 columns, one workgroup of 256, 512 or 1024 threads, streamed beyond 32764), on
+rows whose start is not 16-byte aligned, with special-value rows, against the oracle."""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from synaptik_amd.program import ProgramBuilder
+from tests.gpu_helpers import run_program
+
+pytestmark = pytest.mark.gpu
+
+WIDTHS = [1, 2, 5, 252, 253, 508, 509, 1020, 1021, 2044, 2045, 4092, 4093, 4097, 8188, 8189, 16380,
+          16383, 32764, 32767]
+
+
+@pytest.mark.parametrize("log", [False, True])
+@pytest.mark.parametrize("C", WIDTHS)
+def test_forward(ctx, C, log):
+    print(f"[softmax] C={C} log={log}", flush=True)
+    R = 11
+    rng = np.random.default_rng(C)
+    x = (rng.standard_normal((R, C)) * 3).astype(np.float32)
+    last = C - 1
+    x[1, 0] = np.nan
+    x[2, last] = np.inf
+    x[3, last] = -np.inf
+    x[4, :] = -np.inf
+    x[5, :] = -np.abs(x[5]); x[5, last] = -0.0
+    x[6, :] = -np.abs(x[6]); x[6, 0] = 0.0
+    x[7, 0] = 120.0
+    x[8, :] -= 200.0
+    x[9, 0], x[9, last] = np.nan, np.inf
+    pb = ProgramBuilder()
+    sx, sy, sl = pb.input(R * C), pb.output(R * C), pb.output(R)
+    pb.softmax(sx, sy, R, C, lse=sl, log=log)
+    got, lse = run_program(ctx, pb, [x], [sy, sl])
+    got = got.reshape(R, C)
+    want = oracle.softmax_rows(x, log=log)  # the special-value classes
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    inf = np.isinf(want)
+    assert np.array_equal(got[inf], want[inf])
+    # Finite rows against 64 bits (the oracle's own binary32 Kahan sum is up to 4e-6 off on an
+    # unshifted row): from the rounded difference on, an exponential of one unit, the sum's
+    # rounding and the quotient's (or the logarithm's and the subtraction's).
+    for r in np.flatnonzero(np.isfinite(want if not log else np.where(inf, 0, want)).all(1)):
+        shift = np.float32(0) if np.isneginf(x[r]).any() else x[r].max()
+        d = (x[r] - shift).astype(np.float64)
+        total = np.exp(d).sum()
+        if log:
+            exact, size = d - np.log(total), np.abs(d) + 2 * abs(np.log(total)) + 1
+        else:
+            exact = np.exp(d) / total
+            size = exact + 1e-31
+        fin = np.isfinite(exact)
+        assert np.all(np.abs(got[r][fin] - exact[fin]) <= 4e-7 * size[fin])
+    w = oracle.logsumexp_rows(x)
+    assert np.array_equal(np.isnan(lse), np.isnan(w))
+    assert np.array_equal(lse[np.isinf(w)], w[np.isinf(w)])
+    fin = np.isfinite(w)
+    np.testing.assert_allclose(lse[fin], w[fin], rtol=2e-6, atol=2e-6)
+
+
+@pytest.mark.parametrize("C", WIDTHS)
+def test_backward(ctx, C):
+    print(f"[softmax bwd] C={C}", flush=True)
+    R = 6
+    rng = np.random.default_rng(C + 1)
+    y = oracle.softmax_rows((rng.standard_normal((R, C)) * 2).astype(np.float32))
+    g = rng.standard_normal((R, C)).astype(np.float32)
+    k = rng.standard_normal(R).astype(np.float32)
+    pb = ProgramBuilder()
+    sy, sg, sk = pb.input(R * C), pb.input(R * C), pb.input(R)
+    plain, scaled = pb.output(R * C), pb.output(R * C)
+    pb.softmax_bwd(sy, sg, plain, R, C)
+    pb.softmax_bwd(sy, sg, scaled, R, C, rowscale=sk)
+    a, b = (o.reshape(R, C) for o in run_program(ctx, pb, [y, g, k], [plain, scaled]))
+    want = oracle.softmax_grad_rows(y, g)
+    # y (g - s): s differs by a few units of its last place between sum orders
+    tol = 4e-6 * (np.abs(y) * (np.abs(g) + 1.0)) + 1e-12
+    assert np.all(np.abs(a - want) <= tol)
+    assert np.all(np.abs(b - (want + k[:, None] * y)) <= tol + 2e-7 * np.abs(k[:, None] * y))
