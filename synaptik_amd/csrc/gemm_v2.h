@@ -772,14 +772,13 @@ inline int v2_choose(const GemmParams& p, bool aligned) {
   return !p.transA && p.transB && p.K < 1024 && t64 == 128 ? 0 : 64;
 }
 
-// In-workgroup split-K (KS = 2): fewer than two workgroups per CU and at least four k-tiles per
+// In-workgroup split-K (KS = 2): fewer than two workgroups per CU and at least eight k-tiles per
 // group. Eight waves give each SIMD two, as two four-wave workgroups per CU would, without more
-// partials in HBM (500x1021x509 NN 14.4 us against 17.0 with one group, 1021x617x500 TN 13.9
-// against 16.1). 128x128 tiles only on split-K slices of at least eight k-tiles per group.
+// partials in HBM. 128x128 tiles only on split-K slices.
 inline bool v2_split_in_group(const GemmParams& p, int bt, int64_t tiles, int64_t slices) {
   const int64_t span = p.kchunk > 0 ? p.kchunk : p.K;
   return v2_ks2_enabled() && (bt == 64 || (p.kchunk > 0 && p.partial != nullptr)) &&
-         tiles * slices < 512 && span >= (bt == 64 ? 8 : 16) * V2_BK;
+         tiles * slices < 512 && span >= 16 * V2_BK;
 }
 
 template <bool TA, bool TB, int BT, bool U>
