@@ -6,15 +6,15 @@
 //   logits[r, :]   as gemm_row_dot does: lanes split k in 16-byte steps (fmaf over x, y, z, w),
 //                  the transpose-reduce butterfly over the wave, then + b (the GEMM epilogue);
 //   row_loss[r]    lse - logits[r, t] with the maximum by '>' and the binary64 wave sum of the
-//                  rounded exponentials, as ce_pass1 does (CpuLossReferenceKernel.java:196-218);
-//   dZ[r, :]       (softmax - onehot(t)) * (g / R), the maximum by Math.max, as ce_grad does
+//                  rounded exponentials, as ce_rows_wave does (CpuLossReferenceKernel.java:196-218);
+//   dZ[r, :]       (softmax - onehot(t)) * (g / R), the maximum by Math.max, as ce_rows_wave does
 //                  (LossGradientRules.java:172-240);
 //   dX[r, :]       act_grad(act, dZ[r, :] . W, H[r, :]), each output an fmaf chain over j from +0,
 //                  as gemm_small_k does with the activation-gradient epilogue.
 // Every value is the one the unfused sequence (row-dot GEMM, CE pass 1 and gradient, small-K
 // GEMM) produces, bit for bit: the fusion removes three launches and the logits round trip from
 // the critical path of the backward sweep, nothing else. A second launch (phase 1) finishes the
-// MEAN from the per-row losses with ce_pass1 / ce_finish's grouping: binary64 partials of four
+// MEAN from the per-row losses with ce_rows_wave / ce_finish's grouping: binary64 partials of four
 // consecutive rows, summed over groups in a strided order and a block tree, divided by R.
 #include "common.h"
 #include "gemm_tile.h"

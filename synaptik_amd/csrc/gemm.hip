@@ -202,7 +202,7 @@ namespace {
 //   * Deep problems below that: as many slices as 256 workgroups of 64x64 tiles hold
 //     (64x4096x4096 26.6 in four against 33.3 whole on 32x32 tiles; TN 512x256x8192 26.3 in eight,
 //     600x600x4000 44.0 in two against 60). Deep is K >= 1024 when an operand is M/N-contiguous,
-//     whose 32x32 tiles read poorly (512x1024x1024 TN 16.7 against 56.7), K >= 2048 and 32 tiles
+//     whose 32x32 tiles read poorly (512x1024x1024 TN 16.7 against 22.9), K >= 2048 and 32 tiles
 //     otherwise (K >= 1024 for 128 tiles or more: 512x1024x1024 16.7 against 19.2).
 //   * The others run on 32x32 tiles whose workgroups split K among their waves; slices only up to
 //     192 workgroups (32x1024x1024 8.1 in six against 11.2; 128x1024x512 7.9 whole against 8.4).
