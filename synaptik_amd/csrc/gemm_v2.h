@@ -643,7 +643,13 @@ gemm_f32_v2(GemmParams p) {
         floatx4 v = tile_row(t);
         if constexpr (MODE != 1) {
           if (has_bias) v = floatx4{v[0] + bias[0], v[1] + bias[1], v[2] + bias[2], v[3] + bias[3]};
-          static_for<4>([&](auto c) { v[decltype(c)::value] = apply_act(ACT, v[decltype(c)::value]); });
+          // One binary64 evaluation after the other: interleaved, those of a row batch needed 256
+          // registers and 136 bytes of scratch in every 128x128 kernel, whatever its activation
+          // (195 and none so).
+          static_for<4>([&](auto c) {
+            v[decltype(c)::value] = apply_act(ACT, v[decltype(c)::value]);
+            if constexpr (ACT == ACT_TANH || ACT == ACT_SIGMOID) __builtin_amdgcn_sched_barrier(0);
+          });
         } else {
           const floatx4 y = ya[I];
           static_for<4>([&](auto c) {
