@@ -47,6 +47,10 @@ __device__ __forceinline__ float shifted_exp(float x, float shift) {
   return exp_f32(x - shift);
 }
 
+__device__ __forceinline__ int holds_nan(const float4& v) {
+  return __builtin_isunordered(v.x, v.y) | __builtin_isunordered(v.z, v.w);
+}
+
 // V float4 per thread in registers (C <= V * 4 * SM_NT, C % 4 == 0).
 //
 // The row statistics use the hardware max / min (v_max_f32 / v_min_f32, which skip NaN and need
@@ -243,7 +247,7 @@ struct RowTeam {  // the threads that share a row: a wave, or a workgroup
   struct Shared {
     double d[WAVES];
     float a[WAVES], b[WAVES];
-    int i[WAVES], j[WAVES];
+    int i[WAVES];
   };
   __device__ static __forceinline__ int lane() { return NT == 64 ? threadIdx.x & 63 : threadIdx.x; }
   __device__ static __forceinline__ double sum(double v, Shared& s) {
@@ -257,31 +261,42 @@ struct RowTeam {  // the threads that share a row: a wave, or a workgroup
     for (int w = 0; w < WAVES; ++w) r += s.d[w];
     return r;
   }
-  __device__ static __forceinline__ void extremes(float& mx, float& mn, Shared& s) {
+  // The row's hardware maximum and minimum (both skip NaN) and whether it holds a NaN.
+  __device__ static __forceinline__ void extremes(float& mx, float& mn, int& nan, Shared& s) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       mx = fmaxf(mx, __shfl_xor(mx, o, 64));
       mn = fminf(mn, __shfl_xor(mn, o, 64));
     }
+    nan = __any(nan);
     if constexpr (NT == 64) return;
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) { s.a[threadIdx.x >> 6] = mx; s.b[threadIdx.x >> 6] = mn; }
+    if ((threadIdx.x & 63) == 0) {
+      s.a[threadIdx.x >> 6] = mx;
+      s.b[threadIdx.x >> 6] = mn;
+      s.i[threadIdx.x >> 6] = nan;
+    }
     __syncthreads();
     mx = s.a[0];
     mn = s.b[0];
+    nan = s.i[0];
 #pragma unroll
-    for (int w = 1; w < WAVES; ++w) { mx = fmaxf(mx, s.a[w]); mn = fminf(mn, s.b[w]); }
+    for (int w = 1; w < WAVES; ++w) {
+      mx = fmaxf(mx, s.a[w]);
+      mn = fminf(mn, s.b[w]);
+      nan |= s.i[w];
+    }
   }
-  __device__ static __forceinline__ void either(int& a, int& b, Shared& s) {
+  __device__ static __forceinline__ int any(int a, Shared& s) {
     a = __any(a);
-    b = __any(b);
-    if constexpr (NT == 64) return;
+    if constexpr (NT == 64) return a;
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) { s.i[threadIdx.x >> 6] = a; s.j[threadIdx.x >> 6] = b; }
+    if ((threadIdx.x & 63) == 0) s.i[threadIdx.x >> 6] = a;
     __syncthreads();
-    a = b = 0;
+    a = 0;
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) { a |= s.i[w]; b |= s.j[w]; }
+    for (int w = 0; w < WAVES; ++w) a |= s.i[w];
+    return a;
   }
 };
 
@@ -306,6 +321,7 @@ softmax_fwd_rows(const float* x, float* y, float* lse, int64_t R, int64_t C) {
     const RowGroups view(xr, (int)C);
     float4 v[V];
     float m = -INFINITY, mn = INFINITY;
+    int nan = 0;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
       const int q = tid + i * NT;
@@ -316,6 +332,7 @@ softmax_fwd_rows(const float* x, float* y, float* lse, int64_t R, int64_t C) {
     for (int i = 0; i < V; ++i) {
       const int q = tid + i * NT;
       m = fmaxf(m, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
+      nan |= holds_nan(v[i]);
       if (q < view.groups) {
         if (view.whole(q)) {
           mn = fminf(mn, fminf(fminf(v[i].x, v[i].y), fminf(v[i].z, v[i].w)));
@@ -327,18 +344,18 @@ softmax_fwd_rows(const float* x, float* y, float* lse, int64_t R, int64_t C) {
         }
       }
     }
-    Team::extremes(m, mn, sh);
-    if (m == INFINITY || m == 0.0f) {  // uniform for the row, rare (see softmax_fwd_regs)
-      int nan = 0, pos_zero = 0;
+    Team::extremes(m, mn, nan, sh);
+    // Math.max: a NaN is the maximum, and so the shift. (It also keeps the row off the binary32
+    // exponential, whose result is a finite number for most NaN patterns.)
+    if (nan) {
+      m = NAN;
+    } else if (m == 0.0f) {  // uniform for the row, rare (see softmax_fwd_regs)
+      int pos_zero = 0;
 #pragma unroll
-      for (int i = 0; i < V; ++i) {
-        nan |= (v[i].x != v[i].x) | (v[i].y != v[i].y) | (v[i].z != v[i].z) | (v[i].w != v[i].w);
+      for (int i = 0; i < V; ++i)
         pos_zero |= (__float_as_uint(v[i].x) == 0u) | (__float_as_uint(v[i].y) == 0u) |
                     (__float_as_uint(v[i].z) == 0u) | (__float_as_uint(v[i].w) == 0u);
-      }
-      Team::either(nan, pos_zero, sh);
-      if (nan) m = NAN;
-      else if (m == 0.0f) m = pos_zero ? 0.0f : -0.0f;
+      m = Team::any(pos_zero, sh) ? 0.0f : -0.0f;
     }
     if (m == INFINITY) {
       const float other = LOG ? -INFINITY : 0.0f;

@@ -80,3 +80,27 @@ def test_backward(ctx, C):
     tol = 4e-6 * (np.abs(y) * (np.abs(g) + 1.0)) + 1e-12
     assert np.all(np.abs(a - want) <= tol)
     assert np.all(np.abs(b - (want + k[:, None] * y)) <= tol + 2e-7 * np.abs(k[:, None] * y))
+
+
+# NaN bit patterns: numpy's, the ones whose low payload bits are set, and memory poison. A row is in
+# the binary32 exponential's range but for its NaN.
+NANS = [0x7fc00000, 0x7fc00001, 0x7fffffff, 0xffffffff, 0x7f800001]
+
+
+@pytest.mark.parametrize("log", [False, True])
+@pytest.mark.parametrize("C", [2, 101, 252, 1021, 5003, 20001, 32768, 40000])
+def test_every_nan_pattern_takes_its_row(ctx, C, log):
+    print(f"[softmax nan] C={C} log={log}", flush=True)
+    R = 2 * len(NANS) + 1
+    x = np.random.default_rng(C).standard_normal((R, C)).astype(np.float32)
+    bits = x.view(np.uint32)
+    for i, pattern in enumerate(NANS):
+        bits[i, C // 2] = pattern
+        bits[len(NANS) + i, C - 1] = pattern
+    pb = ProgramBuilder()
+    sx, sy, sl = pb.input(R * C), pb.output(R * C), pb.output(R)
+    pb.softmax(sx, sy, R, C, lse=sl, log=log)
+    got, lse = run_program(ctx, pb, [x], [sy, sl])
+    got = got.reshape(R, C)
+    assert np.all(np.isnan(got[:-1])) and np.all(np.isnan(lse[:-1]))
+    assert np.all(np.isfinite(got[-1])) and np.isfinite(lse[-1])
