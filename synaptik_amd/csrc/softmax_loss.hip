@@ -54,18 +54,17 @@ __device__ __forceinline__ int holds_nan(const float4& v) {
 // V float4 per thread in registers (C <= V * 4 * SM_NT, C % 4 == 0).
 //
 // The row statistics use the hardware max / min (v_max_f32 / v_min_f32, which skip NaN and need
-// not order signed zeros) and restore Math.max semantics where they differ, in a branch taken
-// only by rows whose maximum is +inf or a zero: a NaN anywhere makes the maximum NaN, and a zero
-// maximum is +0 when any element is +0. A row holds -inf exactly when its minimum is -inf.
-// A row with a NaN and no +inf already gives NaN everywhere through the sum, as the reference's
-// NaN shift does.
+// not order signed zeros) and restore Math.max semantics where they differ: a NaN anywhere, which a
+// flag of its own tells, makes the maximum and with it the shift NaN, and a zero maximum is +0 when
+// any element is +0 (a branch taken only by rows whose maximum is a zero). A row holds -inf exactly
+// when its minimum is -inf.
 template <int V>
 __global__ void __launch_bounds__(SM_NT) softmax_fwd_regs(const float* __restrict__ x,
                                                           float* __restrict__ y, float* lse,
                                                           int64_t C, int log_softmax) {
   __shared__ double dl[SM_NT / 64];
   __shared__ float fmx[SM_NT / 64], fmn[SM_NT / 64];
-  __shared__ int il[SM_NT / 64], il2[SM_NT / 64];
+  __shared__ int il[SM_NT / 64], il2[SM_NT / 64];  // (NaN, +0)
   const int64_t r = blockIdx.x;
   const float4* xr = reinterpret_cast<const float4*>(x + r * C);
   float4* yr = reinterpret_cast<float4*>(y + r * C);
@@ -73,11 +72,13 @@ __global__ void __launch_bounds__(SM_NT) softmax_fwd_regs(const float* __restric
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   float4 v[V];
   float m = -INFINITY, mn = INFINITY;
+  int nan = 0;
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     const int c = threadIdx.x + i * SM_NT;
     if (c < C4) {
       v[i] = ld_stream(&xr[c]);
+      nan |= holds_nan(v[i]);
       m = fmaxf(m, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
       mn = fminf(mn, fminf(fminf(v[i].x, v[i].y), fminf(v[i].z, v[i].w)));
     }
@@ -87,36 +88,36 @@ __global__ void __launch_bounds__(SM_NT) softmax_fwd_regs(const float* __restric
     m = fmaxf(m, __shfl_xor(m, o, 64));
     mn = fminf(mn, __shfl_xor(mn, o, 64));
   }
-  if (lane == 0) { fmx[w] = m; fmn[w] = mn; }
+  nan = __any(nan);
+  if (lane == 0) { fmx[w] = m; fmn[w] = mn; il[w] = nan; }
   __syncthreads();
   m = fmx[0];
   mn = fmn[0];
+  nan = il[0];
 #pragma unroll
   for (int i = 1; i < SM_NT / 64; ++i) {
     m = fmaxf(m, fmx[i]);
     mn = fminf(mn, fmn[i]);
+    nan |= il[i];
   }
-  if (m == INFINITY || m == 0.0f) {  // block-uniform, rare
-    int nan = 0, pos_zero = 0;
+  if (nan) {
+    m = NAN;
+  } else if (m == 0.0f) {  // block-uniform, rare
+    int pos_zero = 0;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
       const int c = threadIdx.x + i * SM_NT;
-      if (c < C4) {
-        nan |= (v[i].x != v[i].x) | (v[i].y != v[i].y) | (v[i].z != v[i].z) | (v[i].w != v[i].w);
+      if (c < C4)
         pos_zero |= (__float_as_uint(v[i].x) == 0u) | (__float_as_uint(v[i].y) == 0u) |
                     (__float_as_uint(v[i].z) == 0u) | (__float_as_uint(v[i].w) == 0u);
-      }
     }
-    nan = wave_or(nan);
-    pos_zero = wave_or(pos_zero);
-    if (lane == 0) { il[w] = nan; il2[w] = pos_zero; }
+    pos_zero = __any(pos_zero);
+    if (lane == 0) il2[w] = pos_zero;
     __syncthreads();
-    nan = 0;
     pos_zero = 0;
 #pragma unroll
-    for (int i = 0; i < SM_NT / 64; ++i) { nan |= il[i]; pos_zero |= il2[i]; }
-    if (nan) m = NAN;
-    else if (m == 0.0f) m = pos_zero ? 0.0f : -0.0f;
+    for (int i = 0; i < SM_NT / 64; ++i) pos_zero |= il2[i];
+    m = pos_zero ? 0.0f : -0.0f;
   }
   if (m == INFINITY) {
     const float other = log_softmax ? -INFINITY : 0.0f;

@@ -88,7 +88,7 @@ NANS = [0x7fc00000, 0x7fc00001, 0x7fffffff, 0xffffffff, 0x7f800001]
 
 
 @pytest.mark.parametrize("log", [False, True])
-@pytest.mark.parametrize("C", [2, 101, 252, 1021, 5003, 20001, 32768, 40000])
+@pytest.mark.parametrize("C", [2, 101, 252, 512, 1021, 2044, 4096, 5003, 20001, 32768, 40000])
 def test_every_nan_pattern_takes_its_row(ctx, C, log):
     print(f"[softmax nan] C={C} log={log}", flush=True)
     R = 2 * len(NANS) + 1
