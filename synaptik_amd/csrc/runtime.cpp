@@ -241,9 +241,10 @@ struct Lease {
   std::map<std::vector<void*>, hipGraphExec_t> graph_cache;
   std::vector<std::vector<void*>> graph_order;
   bool graphs_ok = true;  // a capture failed on this lease: launch step by step from then on
-  // Every run ends with a kernel that copies the status word to host_status and clears it, so
-  // the next run on this lease starts from a clear word. Until a run has completed that way (a
-  // new lease, a failed launch or execution) the next run clears the word first.
+  // A run that can flag the status word ends with a kernel that copies the word to host_status and
+  // clears it, and no step of any other run touches it (Program::publishes), so the next run on
+  // this lease starts from a clear word. Until a run has completed (a new lease, a failed launch or
+  // execution) the next run clears the word first.
   bool status_clear = false;
 };
 
@@ -271,8 +272,8 @@ struct Program {
   // Whether a run ends with the publication kernel: not when no step touches the status word, no
   // step is folded and there is no step counter to commit (inference, a layer, softmax, chains
   // and reductions), where it would copy a word that stays clear. It is a launch of 3 to 4 us on
-  // MI355X: a batch-1 inference of three GEMMs
-  // took 29.1 us with it and 24.5 without.
+  // MI355X: a batch-1 inference of three GEMMs took 29.1 us with it and 24.5 without. A program
+  // none of whose steps launches anything (extents of zero) keeps it, so that no run is empty.
   bool publishes = true;
   bool folded(size_t j) const {
     return (int64_t)j == folded_finish || (int64_t)j == folded_opt;
@@ -917,6 +918,19 @@ Access step_access(const Step& st) {
       W(-2);
   }
   return x;
+}
+// Whether a step that does not touch the status word launches a kernel: not one whose result has
+// no elements.
+bool step_launches(const StepRecord& r) {
+  const int64_t* a = r.iarg;
+  switch (r.opcode) {
+    case OP_GEMM: case OP_POINTWISE: case OP_SOFTMAX_BWD: case OP_LSE_BWD: case OP_TRANSPOSE:
+      return a[0] > 0 && a[1] > 0;
+    case OP_COLSUM: return a[1] > 0;
+    case OP_ROW_REDUCE: case OP_SOFTMAX: case OP_CE_HEAD: case OP_FILL: case OP_COPY:
+      return a[0] > 0;
+    default: return true;  // (REDUCE_ALL, MSE)
+  }
 }
 bool accesses_conflict(const Access& a, const Access& b) {
   auto meet = [](const std::vector<int32_t>& u, const std::vector<int32_t>& v) {
@@ -1851,11 +1865,14 @@ int32_t decode_image(const void* image, uint64_t image_bytes, Program* pr) {
   off += ((scratch_doubles * 8 + 255) / 256) * 256;
   plan_fold(pr);
   plan_streams(pr);
-  pr->publishes = pr->steps.empty() || pr->folded_finish >= 0 || pr->folded_opt >= 0;
+  pr->publishes = pr->folded_finish >= 0 || pr->folded_opt >= 0;
+  bool launches = false;
   for (const Step& st : pr->steps) {
     const Access x = step_access(st);
     pr->publishes |= x.status_or || x.status_read;  // (a step commit reads the word)
+    launches |= step_launches(st.rec);
   }
+  pr->publishes |= !launches;
   pr->scratch_side_off = off;
   if (pr->side_steps > 0) off += ((scratch_doubles * 8 + 255) / 256) * 256;
   pr->internal_offset.assign(h.n_slots, 0);

@@ -44,3 +44,36 @@ def test_run_without_publication(ctx, mode):
         assert np.all(np.abs(by.download(np.float32, R) - want) <= 3 * 2.0 ** -23 * want)
     prog.close()
     flagging.close()
+
+
+@pytest.mark.parametrize("mode", ["graph", "direct", "profiled", "async", "static"])
+def test_run_of_steps_without_elements(ctx, mode):
+    """Nothing but steps of extent zero: such a program still publishes, so that its run, and its
+    captured graph, hold a launch. The outputs stay as they were."""
+    pb = ProgramBuilder()
+    x, y, z = pb.input(8), pb.output(8), pb.output(8)
+    pb.softmax(x, y, 0, 8)
+    pb.row_reduce(x, y, 0, 8, "max")
+    pb.colsum(x, y, 1, 0, ldx=8)
+    pb.gemm(x, x, y, 0, 2, 4)
+    pb.softmax_bwd(x, x, z, 4, 0)
+    pb.lse_bwd(x, x, z, 0, 4)
+    pb.pointwise(0, 4, [x], [z], [("load", 0, 0, 0, 0, 0.0), ("neg", 1, 0, 0, 0, 0.0),
+                                  ("store", 0, 1, 0, 0, 0.0)])
+    pb.transpose(x, z, 0, 4)
+    pb.fill(z, 0)
+    pb.copy(x, z, 0)
+    prog = HipProgram(ctx, pb.image())
+    prog.set_graph_mode(mode == "graph")
+    prog.set_profiling(mode == "profiled")
+    data = np.arange(8, dtype=np.float32)
+    bx, by, bz = ctx.upload(data + 10), ctx.upload(data), ctx.upload(-data)
+    for _ in range(3):
+        if mode == "async":
+            prog.run_async([bx], [by, bz])
+            prog.wait()
+        else:
+            (prog.run_static if mode == "static" else prog.run)([bx], [by, bz])
+        assert np.array_equal(by.download(np.float32, 8), data)
+        assert np.array_equal(bz.download(np.float32, 8), -data)
+    prog.close()
