@@ -37,6 +37,9 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
 
 constexpr int DK = 16;  // depth of a step
+// Tiles in the grid's first dimension, which holds fewer than 2^32 threads; the rest go to planes
+// along z.
+constexpr uint32_t DIRECT_GRID_X = 1 << 20;
 
 // One operand's fragments of a wave tile.
 template <bool KMAJ, int NB>
@@ -120,7 +123,9 @@ struct DirectCfg {
   static constexpr int EC = T < 4 ? T : 4;         // passes whose loads go out together
 };
 
-template <bool KA, bool KB, int NB, int MW, int NW, int KW>
+// PLANES: the tiles beyond DIRECT_GRID_X lie in further planes of the grid (of their own, because
+// the test costs a product of a million short rows 1%).
+template <bool KA, bool KB, int NB, int MW, int NW, int KW, bool PLANES>
 __global__ void __launch_bounds__(64 * MW * NW * KW) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_direct(GemmParams p) {
   using Cfg = DirectCfg<NB, MW, NW, KW>;
@@ -128,8 +133,10 @@ gemm_direct(GemmParams p) {
   __shared__ __attribute__((aligned(16))) float stage[KW * TM * TN];
 
   const int tilesM = (int)((p.M + TM - 1) / TM), tilesN = (int)((p.N + TN - 1) / TN);
+  const int id = (int)(blockIdx.x + (PLANES ? blockIdx.z * DIRECT_GRID_X : 0u));
+  if (PLANES && id >= tilesM * tilesN) return;  // the last plane ends short
   int tm, tn;
-  tile_of(blockIdx.x, tilesM, tilesN, tm, tn);
+  tile_of(id, tilesM, tilesN, tm, tn);
   const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int kw = wave / (MW * NW), wm = (wave / NW) % MW, wn = wave % NW;
@@ -404,13 +411,15 @@ gemm_direct(GemmParams p) {
   }
 }
 
-template <int NB, int MW, int NW, int KW, bool TA, bool TB>
+template <int NB, int MW, int NW, int KW, bool PLANES, bool TA, bool TB>
 hipError_t launch_direct_cfg(const GemmParams& p, hipStream_t s) {
   using Cfg = DirectCfg<NB, MW, NW, KW>;
   const int64_t tm = (p.M + Cfg::TM - 1) / Cfg::TM, tn = (p.N + Cfg::TN - 1) / Cfg::TN;
   const int64_t slices = p.kchunk > 0 ? (p.K + p.kchunk - 1) / p.kchunk : 1;
   g_colsum_rows = tm;
-  hipLaunchKernelGGL((gemm_direct<!TA, TB, NB, MW, NW, KW>), dim3((unsigned)(tm * tn), (unsigned)slices),
+  const int64_t x = PLANES ? DIRECT_GRID_X : tm * tn;
+  hipLaunchKernelGGL((gemm_direct<!TA, TB, NB, MW, NW, KW, PLANES>),
+                     dim3((unsigned)x, (unsigned)slices, (unsigned)((tm * tn + x - 1) / x)),
                      dim3(Cfg::NT), 0, s, p);
   return hipGetLastError();
 }
@@ -424,8 +433,10 @@ inline bool direct_wide(const GemmParams& p) {
 
 template <bool TA, bool TB>
 hipError_t launch_direct(const GemmParams& p, hipStream_t s) {
-  return direct_wide(p) ? launch_direct_cfg<2, 2, 2, 2, TA, TB>(p, s)
-                        : launch_direct_cfg<2, 1, 1, 8, TA, TB>(p, s);
+  if (!direct_wide(p)) return launch_direct_cfg<2, 1, 1, 8, false, TA, TB>(p, s);
+  return ((p.M + 63) / 64) * ((p.N + 63) / 64) <= DIRECT_GRID_X
+             ? launch_direct_cfg<2, 2, 2, 2, false, TA, TB>(p, s)
+             : launch_direct_cfg<2, 2, 2, 2, true, TA, TB>(p, s);
 }
 
 }  // namespace

@@ -741,6 +741,9 @@ inline bool v2_aligned(const GemmParams& p, bool va, bool vb) {
          (p.mode == 0 || (al(p.aux) && p.ldaux % 4 == 0)) && (p.mode != 2 || al(p.dz));
 }
 
+// A launch holds fewer than 2^32 threads in each dimension.
+constexpr int64_t V2_MAX_TILES = (1LL << 32) / V2_NT;
+
 // Tile edge of the direct-to-LDS kernel for a GEMM, or 0 when gemm_direct runs it. Figures: us on
 // MI355X for one GEMM, sizes M x N x K.
 //   * Whole K. A CU works through its 128x128 tiles two at a time, so the time goes with
@@ -754,26 +757,31 @@ inline bool v2_aligned(const GemmParams& p, bool va, bool vb) {
 //     holds for 128 tiles too (512x1024x400 10.1 against 13.0; NN 14.6 against 12.8).
 //   * Split-K slices (gemm_slices): 128 where the plan counted in 128x128 tiles, 64 for the other
 //     plans that reach 128 workgroups; gemm_direct for the rest.
+//   * Operands of any size, as long as the lane offsets inside a tile fit 32 bits (origins and
+//     results are addressed with 64): a leading dimension of 8.4 million for K-contiguous operands,
+//     34 million for the others. 65536x1024x32768 NN 28.8 ms here against 79.9 on gemm_direct, TN
+//     1024x256x2097152 10.1 against 54.7.
 // TAIL variants run when M, N or K (or the slice) is not a whole number of tiles.
 inline int v2_choose(const GemmParams& p, bool aligned) {
-  // the moved last tile of the U form needs a whole tile of its operand
-  auto fits = [&](int bt) {
-    return aligned || ((!p.transA || p.M >= bt) && (p.transB || p.N >= bt));
-  };
   if (p.K < 4 || (p.kchunk > 0 && (p.kchunk % V2_BK != 0 || p.partial == nullptr))) return 0;
-  const int64_t ld = std::max(p.lda, p.ldb);
-  if ((p.M + 128) * ld >= (1LL << 31) || (p.N + 128) * ld >= (1LL << 31) ||
-      (p.K + 128) * ld >= (1LL << 31))
-    return 0;
   const int64_t slices = p.kchunk > 0 ? (p.K + p.kchunk - 1) / p.kchunk : 1;
   const int64_t t128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
   const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
-  if (t64 >= (1LL << 31) || slices >= 65536) return 0;
+  auto fits = [&](int bt) {
+    // the moved last tile of the U form needs a whole tile of its operand
+    return (aligned || ((!p.transA || p.M >= bt) && (p.transB || p.N >= bt))) &&
+           v2_offsets_fit(p.M, p.K, p.lda, !p.transA, bt) &&
+           v2_offsets_fit(p.N, p.K, p.ldb, p.transB, bt) &&
+           (bt == 64 ? t64 : t128) < V2_MAX_TILES;
+  };
+  if (slices >= 65536) return 0;
   if (p.kchunk > 0) {
-    if (aligned && t64 >= 256 && t128 * slices >= 256) return 128;
+    if (aligned && t64 >= 256 && t128 * slices >= 256 && fits(128)) return 128;
     return t64 * slices >= 128 && fits(64) ? 64 : 0;
   }
-  if (t128 >= 256 && 4 * ((t128 + 255) / 256) <= (t64 + 255) / 256 && fits(128)) return 128;
+  if (t128 >= 256 && (4 * ((t128 + 255) / 256) <= (t64 + 255) / 256 || t64 >= V2_MAX_TILES) &&
+      fits(128))
+    return 128;
   if (t64 < 128 || !fits(64)) return 0;
   return !p.transA && p.transB && p.K < 1024 && t64 == 128 ? 0 : 64;
 }

@@ -30,4 +30,12 @@ __host__ __device__ constexpr int v2_mnmaj_src(int q, int cpr) {
   return (q / cpr) * cpr + ((q % cpr) ^ ((((q / cpr) >> 2) & 3) << 2));
 }
 
+// Whether the copies' lane offsets, unsigned 32-bit byte offsets from a tile's 64-bit origin, reach
+// every element of an operand that a lane copies: `rows` is its M or N extent, `ld` its leading
+// dimension. (Lanes whose rows or k lie outside the operand copy nothing.)
+constexpr bool v2_offsets_fit(long long rows, long long K, long long ld, bool k_contiguous, int bt) {
+  const long long lines = k_contiguous ? (rows < bt ? rows : bt) : (K < 32 ? K : 32);
+  return (lines - 1) * ld + (k_contiguous ? 32 : bt) <= (1LL << 30);  // floats
+}
+
 }  // namespace shk

@@ -3,7 +3,8 @@
 // fragment addressing (source -> LDS offset) are inverse bijections over a stage; the kernel's
 // fragment offsets (a per-lane base plus compile-time block / k-row offsets, as gemm_v2.h forms
 // them) equal the layout function; every 16-lane phase of a K-contiguous ds_read_b128 covers 16
-// distinct 16-byte bank groups and every M/N-contiguous ds_read_b32 covers 64 distinct banks.
+// distinct 16-byte bank groups and every M/N-contiguous ds_read_b32 covers 64 distinct banks; the rule
+// for the copies' 32-bit offsets is exact.
 // Prints "ok" or the first failure.
 #include <cstdio>
 #include <vector>
@@ -65,8 +66,37 @@ static int check(int BT) {
   return 0;
 }
 
+// v2_offsets_fit against the offsets gemm_v2.h forms: accepted when the last byte of every copied
+// chunk lies within 2^32 of the tile origin, refused when one does not, however large the operand.
+static int check_offsets() {
+  const long long rows[] = {1, 17, 64, 100, 128, 1024, 2097152, 65536}, depths[] = {4, 31, 32, 1024, 2097152};
+  const long long lds[] = {4, 1024, 32768, 1 << 20, 8000000, 8454000, 8455000, 16777216, 17043000, 17044000,
+                           34636000, 34637000, 1 << 28};
+  for (int BT : {64, 128})
+    for (long long R : rows)
+      for (long long K : depths)
+        for (long long ld : lds)
+          for (int kmaj = 0; kmaj < 2; ++kmaj) {
+            long long last = 0;  // one past the last byte
+            for (int q = 0; q < BT * 8; ++q) {
+              const int t = kmaj ? v2_kmaj_src(q) : v2_mnmaj_src(q, BT / 4);
+              const int line = kmaj ? t >> 3 : t / (BT / 4), c = kmaj ? t & 7 : t % (BT / 4);
+              if (line >= (kmaj ? R : K)) continue;  // outside the operand: not copied
+              const long long end = (line * ld + 4 * c) * 4 + 16;
+              if (end > last) last = end;
+            }
+            if (v2_offsets_fit(R, K, ld, kmaj != 0, BT) != (last <= (1LL << 32)))
+              return fail("offsets", BT, (int)R, (int)(ld >> 10), kmaj);
+          }
+  // 2^31 elements and more: activations, a vocabulary head, a contraction over many rows
+  if (!v2_offsets_fit(2097152, 1024, 1024, true, 128) || !v2_offsets_fit(65536, 32768, 32768, true, 128) ||
+      !v2_offsets_fit(1024, 2097152, 1024, false, 64))
+    return fail("large operands", 0, 0, 0, 0);
+  return 0;
+}
+
 int main() {
-  if (check(128) || check(64)) return 1;
+  if (check(128) || check(64) || check_offsets()) return 1;
   printf("ok\n");
   return 0;
 }

@@ -6,6 +6,7 @@ bit, whatever the order of the sums; each epilogue is checked the same way."""
 import numpy as np
 import pytest
 
+from synaptik_amd.native import HipProgram
 from synaptik_amd.program import ProgramBuilder
 from tests.gpu_helpers import run_program
 
@@ -113,3 +114,57 @@ def test_infinities_stay_in_their_rows(ctx):
         rest = np.delete(np.arange(M), 5)
         want = np.broadcast_to(A[rest].sum(1, dtype=np.float64)[:, None], (M - 1, N))
         assert np.array_equal(got[rest], want.astype(np.float32))
+
+
+
+def _run_periodic(ctx, M, N, K, ta, tb, block, B):
+    """C = op(A).op(B) with A the rows of `block` over and over, uploaded one repetition a time."""
+    rows, width = (K, M) if ta else (M, K)
+    a = ctx.buffer(4 * rows * width)
+    for r in range(0, rows, len(block)):
+        a.upload(block[:rows - r], 4 * r * width)
+    pb = ProgramBuilder()
+    xa, xb, xc = pb.input(M * K), pb.input(K * N), pb.output(M * N)
+    pb.gemm(xa, xb, xc, M, N, K, trans_a=ta, trans_b=tb)
+    prog = HipProgram(ctx, pb.image())
+    c = ctx.buffer(4 * M * N)
+    prog.run([a, ctx.upload(np.ascontiguousarray(B.T) if tb else B)], [c])
+    prog.close()
+    return c.download(np.float32, M * N).reshape(M, N)
+
+
+def _assert_periodic(got, block, B):
+    want = (block.astype(np.float64) @ B.astype(np.float64)).astype(np.float32)
+    for r in range(0, len(got), len(want)):
+        assert np.array_equal(got[r:r + len(want)], want[:len(got) - r]), r
+
+
+@pytest.mark.parametrize("M,N,K,ta,tb", [
+    (2097153, 64, 1024, False, True),    # aligned operands, ragged M
+    (2097153, 68, 1027, False, False),   # the unaligned form
+    (1024, 96, 2097155, True, False),    # a contraction over as many rows, in slices
+])
+def test_operands_beyond_two_to_the_31_elements(ctx, M, N, K, ta, tb):
+    print(f"[gemm] large {M}x{N}x{K} ta={ta} tb={tb}", flush=True)
+    rng = np.random.default_rng(N)
+    block = rng.integers(-1, 2, (40009, M if ta else K)).astype(np.float32)
+    B = rng.integers(-1, 2, (K, N), dtype=np.int8).astype(np.float32)
+    got = _run_periodic(ctx, M, N, K, ta, tb, block, B)
+    if not ta:
+        _assert_periodic(got, block, B)
+        return
+    folded = np.zeros((len(block), N))  # the rows of B that meet one row of the block
+    for r in range(0, K, len(block)):
+        folded[:min(len(block), K - r)] += B[r:r + len(block)]
+    # whole numbers below 2^24: exact in any order
+    assert np.array_equal(got, (block.T.astype(np.float64) @ folded).astype(np.float32))
+
+
+def test_more_tiles_than_one_grid_plane(ctx):
+    """More than 2^20 64x64 tiles of the register kernel: its grid has planes."""
+    M, N, K = 64 * (1 << 20) + 65, 17, 17
+    print(f"[gemm] planes {M}x{N}x{K}", flush=True)
+    rng = np.random.default_rng(17)
+    block = rng.integers(-3, 4, (1000003, K)).astype(np.float32)
+    B = rng.integers(-3, 4, (K, N)).astype(np.float32)
+    _assert_periodic(_run_periodic(ctx, M, N, K, False, False, block, B), block, B)
