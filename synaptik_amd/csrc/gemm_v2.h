@@ -52,8 +52,10 @@ constexpr int V2_GROUP = 4, V2_GROUP64 = 2;
 
 // U (unaligned): operands of any alignment, leading dimension, K, M and N. A 16-byte copy may start
 // at any float of the operand; what it may not do is take in floats beyond the operand's row, so
-//   * the last tile of an M/N-contiguous operand is moved back to end with the operand (its extent
-//     is at least BT) and the epilogue leaves out the rows or columns the tile before it stores;
+//   * the last tile of an M/N-contiguous operand is moved back to end with the operand, and the
+//     epilogue leaves out the rows or columns the tile before it stores. An operand of less than a
+//     tile stays where it is: its last chunk at each k takes in up to three floats of the row after
+//     (they reach only results that are not stored), and at the last k it is loaded float by float;
 //   * the chunk of a K-contiguous row that K cuts is loaded float by float (once per tile).
 template <int BT, bool U>
 struct V2Cfg {
@@ -107,8 +109,13 @@ struct V2Loader {
     const uint32_t dst =
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)lds + I * 4096u + wdst;
     // a whole tile row-range and a whole k-tile (uniform) need no per-lane bounds
-    if (!TAIL || (rows_left >= BT && k_left >= V2_BK) ||
-        (vrow[I] < rows_left && vk[I] + (U && KMAJ ? 3 : 0) < k_left)) {
+    const bool inside = vrow[I] < rows_left && vk[I] < k_left;
+    // U: a chunk cut by the end of a K-contiguous row is loaded float by float; one cut by the end of
+    // an M/N-contiguous row takes in floats of the row after it, unless there is none
+    const bool whole = !U ? inside
+                       : KMAJ ? inside && vk[I] + 3 < k_left
+                              : inside && (vrow[I] + 3 < rows_left || vk[I] + 1 < k_left);
+    if (!TAIL || (rows_left >= BT && k_left >= V2_BK) || whole) {
       asm volatile("global_load_lds_dwordx4 %0, %1"
                    :
                    : "v"(voff[I]), "s"(tile), "{m0}"(dst)
@@ -116,11 +123,12 @@ struct V2Loader {
     } else {
       const int w = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
       floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (U && KMAJ && vrow[I] < rows_left && vk[I] < k_left) {  // the chunk that K cuts
+      if (U && inside) {  // a cut chunk
         const float* src = tile + voff[I] / 4;
+        const int left = KMAJ ? k_left - vk[I] : rows_left - vrow[I];
         v[0] = src[0];
-        if (vk[I] + 1 < k_left) v[1] = src[1];
-        if (vk[I] + 2 < k_left) v[2] = src[2];
+        if (left > 1) v[1] = src[1];
+        if (left > 2) v[2] = src[2];
       }
       *reinterpret_cast<floatx4*>(lds + (I * 4 + w) * 256 + lane * 4) = v;
     }
@@ -263,8 +271,8 @@ gemm_f32_v2(GemmParams p) {
   tile_of(blockIdx.x, tilesM, tilesN, tm, tn);
   // first row and column this tile stores, and its origin (U: moved back at the operand's end)
   const int64_t m_first = (int64_t)tm * BT, n_first = (int64_t)tn * BT;
-  const int64_t m0 = U && !KA ? std::min<int64_t>(m_first, p.M - BT) : m_first;
-  const int64_t n0 = U && !KB ? std::min<int64_t>(n_first, p.N - BT) : n_first;
+  const int64_t m0 = U && !KA && p.M > BT ? std::min<int64_t>(m_first, p.M - BT) : m_first;
+  const int64_t n0 = U && !KB && p.N > BT ? std::min<int64_t>(n_first, p.N - BT) : n_first;
   const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, g = lane >> 4;
@@ -761,15 +769,25 @@ constexpr int64_t V2_MAX_TILES = (1LL << 32) / V2_NT;
 //     results are addressed with 64): a leading dimension of 8.4 million for K-contiguous operands,
 //     34 million for the others. 65536x1024x32768 NN 28.8 ms here against 79.9 on gemm_direct, TN
 //     1024x256x2097152 10.1 against 54.7.
+//   * Unaligned M/N-contiguous operands of less than a tile (times of whole calls): with 33 to 63
+//     rows or columns from 512 tiles on, from 256 with K > 64 (30001x63x1021 NN 53 here, 96 and 106
+//     on gemm_direct's 32x32 and 64x64 tiles, TN 53 against 109 and 121; 30001x63x33 NN 20.1 against
+//     25.0 and 19.6). With fewer only TN, whose fragments gemm_direct reads 8 bytes at a time, from
+//     K = 128 on (17x30001x509 TN 38.9 against 52.6; NN 30001x17x509 40.7 against 34.6).
 // TAIL variants run when M, N or K (or the slice) is not a whole number of tiles.
 inline int v2_choose(const GemmParams& p, bool aligned) {
   if (p.K < 4 || (p.kchunk > 0 && (p.kchunk % V2_BK != 0 || p.partial == nullptr))) return 0;
   const int64_t slices = p.kchunk > 0 ? (p.K + p.kchunk - 1) / p.kchunk : 1;
   const int64_t t128 = ((p.M + 127) / 128) * ((p.N + 127) / 128);
   const int64_t t64 = ((p.M + 63) / 64) * ((p.N + 63) / 64);
+  // U: an M/N-contiguous operand's extent
+  auto enough = [&](int64_t extent, int bt) {
+    if (aligned || extent >= bt) return true;
+    if (bt != 64 || p.kchunk > 0 || t64 < 256) return false;
+    return extent > 32 ? p.K > 64 || t64 >= 512 : p.transA && !p.transB && p.K >= 128;
+  };
   auto fits = [&](int bt) {
-    // the moved last tile of the U form needs a whole tile of its operand
-    return (aligned || ((!p.transA || p.M >= bt) && (p.transB || p.N >= bt))) &&
+    return (!p.transA || enough(p.M, bt)) && (p.transB || enough(p.N, bt)) &&
            v2_offsets_fit(p.M, p.K, p.lda, !p.transA, bt) &&
            v2_offsets_fit(p.N, p.K, p.ldb, p.transB, bt) &&
            (bt == 64 ? t64 : t128) < V2_MAX_TILES;

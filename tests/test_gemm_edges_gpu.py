@@ -50,6 +50,25 @@ def test_exact_products(ctx, M, N, K, ta, tb, pad):
     assert np.array_equal(got.reshape(M, N), want)
 
 
+# M/N-contiguous operands of less than a 64-wide tile, many tiles along the other extent: LDS tiles
+# whose chunks run past the operand's row, 64x64 register tiles (the last three), by layout and K
+NARROW = [(33, 17000, 67), (17000, 63, 97), (61, 16500, 520), (20, 16500, 130), (33000, 33, 33),
+          (16500, 17, 19), (31, 16500, 19), (16385, 32, 127)]
+
+
+@pytest.mark.parametrize("pad", [0, 1])
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("M,N,K", NARROW)
+def test_narrow_operands(ctx, M, N, K, ta, tb, pad):
+    test_exact_products(ctx, M, N, K, ta, tb, pad)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("M,N,K", [(33, 17000, 67), (17000, 61, 97), (16500, 17, 19)])
+def test_narrow_epilogues(ctx, M, N, K, ta, tb):
+    test_epilogues(ctx, M, N, K, ta, tb)
+
+
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
 @pytest.mark.parametrize("M,N,K", [(33, 47, 31), (97, 301, 515), (1025, 513, 67), (2047, 2047, 35),
                                    (385, 387, 2051)])
