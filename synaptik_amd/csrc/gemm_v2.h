@@ -72,7 +72,8 @@ struct V2Cfg {
 
 // Per-lane source offsets (bytes, relative to the tile origin) of the NI 16-byte copies this
 // thread issues per operand per k-tile, where they land, and (TAIL) the chunk's coordinates.
-template <bool KMAJ, int BT, bool TAIL, bool U>
+// CUT: an M/N-contiguous operand of less than a tile (see U above).
+template <bool KMAJ, int BT, bool TAIL, bool U, bool CUT>
 struct V2Loader {
   using Cfg = V2Cfg<BT, U>;
   uint32_t voff[Cfg::NI];
@@ -109,13 +110,9 @@ struct V2Loader {
     const uint32_t dst =
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)lds + I * 4096u + wdst;
     // a whole tile row-range and a whole k-tile (uniform) need no per-lane bounds
-    const bool inside = vrow[I] < rows_left && vk[I] < k_left;
-    // U: a chunk cut by the end of a K-contiguous row is loaded float by float; one cut by the end of
-    // an M/N-contiguous row takes in floats of the row after it, unless there is none
-    const bool whole = !U ? inside
-                       : KMAJ ? inside && vk[I] + 3 < k_left
-                              : inside && (vrow[I] + 3 < rows_left || vk[I] + 1 < k_left);
-    if (!TAIL || (rows_left >= BT && k_left >= V2_BK) || whole) {
+    if (!TAIL || (rows_left >= BT && k_left >= V2_BK) ||
+        (vrow[I] < rows_left && vk[I] + (U && KMAJ ? 3 : 0) < k_left &&
+         (!CUT || vrow[I] + 3 < rows_left || vk[I] + 1 < k_left))) {
       asm volatile("global_load_lds_dwordx4 %0, %1"
                    :
                    : "v"(voff[I]), "s"(tile), "{m0}"(dst)
@@ -123,12 +120,17 @@ struct V2Loader {
     } else {
       const int w = (threadIdx.x >> 6) & 3, lane = threadIdx.x & 63;
       floatx4 v = floatx4{0.f, 0.f, 0.f, 0.f};
-      if (U && inside) {  // a cut chunk
+      if (U && KMAJ && vrow[I] < rows_left && vk[I] < k_left) {  // the chunk that K cuts
         const float* src = tile + voff[I] / 4;
-        const int left = KMAJ ? k_left - vk[I] : rows_left - vrow[I];
         v[0] = src[0];
-        if (left > 1) v[1] = src[1];
-        if (left > 2) v[2] = src[2];
+        if (vk[I] + 1 < k_left) v[1] = src[1];
+        if (vk[I] + 2 < k_left) v[2] = src[2];
+      }
+      if (CUT && vrow[I] < rows_left && vk[I] < k_left) {  // the cut chunk of the last k
+        const float* src = tile + voff[I] / 4;
+        v[0] = src[0];
+        if (vrow[I] + 1 < rows_left) v[1] = src[1];
+        if (vrow[I] + 2 < rows_left) v[2] = src[2];
       }
       *reinterpret_cast<floatx4*>(lds + (I * 4 + w) * 256 + lane * 4) = v;
     }
@@ -249,7 +251,9 @@ __device__ __forceinline__ void v2_barrier() {
 // in LDS and share the epilogue, each value the sum group 0 + group 1 (a fixed order), stored as
 // the result or, for a slice, as the slice's partial. It gives each SIMD two waves on problems
 // with too few tiles for two workgroups per CU, without more partials in HBM or a second launch.
-template <bool KA, bool KB, int BT, bool TAIL, int KS, bool U = false>
+// CUT: a U kernel for an M/N-contiguous operand of less than a tile (a form of its own: the test of
+// each chunk costs the others 4%).
+template <bool KA, bool KB, int BT, bool TAIL, int KS, bool U = false, bool CUT = false>
 __global__ void __launch_bounds__(V2_NT * KS) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_f32_v2(GemmParams p) {
   static_assert(!U || TAIL, "operands of any alignment have edges");
@@ -271,8 +275,10 @@ gemm_f32_v2(GemmParams p) {
   tile_of(blockIdx.x, tilesM, tilesN, tm, tn);
   // first row and column this tile stores, and its origin (U: moved back at the operand's end)
   const int64_t m_first = (int64_t)tm * BT, n_first = (int64_t)tn * BT;
-  const int64_t m0 = U && !KA && p.M > BT ? std::min<int64_t>(m_first, p.M - BT) : m_first;
-  const int64_t n0 = U && !KB && p.N > BT ? std::min<int64_t>(n_first, p.N - BT) : n_first;
+  const int64_t m0 =
+      U && !KA && !(CUT && p.M < BT) ? std::min<int64_t>(m_first, p.M - BT) : m_first;
+  const int64_t n0 =
+      U && !KB && !(CUT && p.N < BT) ? std::min<int64_t>(n_first, p.N - BT) : n_first;
   const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, g = lane >> 4;
@@ -295,8 +301,8 @@ gemm_f32_v2(GemmParams p) {
   const float* b_tile = KB ? p.B + n0 * p.ldb + k_begin : p.B + n0 + k_begin * p.ldb;
   const int64_t a_step = KA ? V2_BK : V2_BK * p.lda;
   const int64_t b_step = KB ? V2_BK : V2_BK * p.ldb;
-  V2Loader<KA, BT, TAIL, U> la;
-  V2Loader<KB, BT, TAIL, U> lb;
+  V2Loader<KA, BT, TAIL, U, CUT && !KA> la;
+  V2Loader<KB, BT, TAIL, U, CUT && !KB> lb;
   la.init(p.lda);
   lb.init(p.ldb);
 
@@ -761,8 +767,11 @@ constexpr int64_t V2_MAX_TILES = (1LL << 32) / V2_NT;
 //     5120x2048x1024 180 against 152, 4096x1536x1024 121 against 98; 4096x1024x1024 65.2 against
 //     65.9, 4095^3 1038 against 1068.
 //   * 64 needs 128 tiles; below that a workgroup of gemm_direct's 32x32 tiles finishes sooner
-//     (256x1024x1024 NT 11.6 against 18.9). With both operands K-contiguous and K < 1024 that
-//     holds for 128 tiles too (512x1024x400 10.1 against 13.0; NN 14.6 against 12.8).
+//     (256x1024x1024 NT 11.6 against 18.9). At 128 tiles, two 32x32 workgroups a CU, that still
+//     holds with both operands K-contiguous and K < 1024 (whole calls: 512x1024x400 NT 20.4 against
+//     23.5, 512x1024x1000 28.6 against 32.6). The other layouts lie on either side (NN 512x1024x400
+//     22.0 against 23.4 and 500x1021x509 24.4 against 27.4; 512x1024x512 24.0 against 22.6,
+//     64x8192x256 19.4 against 18.7, TN 1021x500x617 27.7 against 26.9) and keep the LDS tiles.
 //   * Split-K slices (gemm_slices): 128 where the plan counted in 128x128 tiles, 64 for the other
 //     plans that reach 128 workgroups; gemm_direct for the rest.
 //   * Operands of any size, as long as the lane offsets inside a tile fit 32 bits (origins and
@@ -821,6 +830,15 @@ hipError_t launch_v2_bt(const GemmParams& p, hipStream_t s) {
   const bool ks2 = !(U && BT == 128) && v2_split_in_group(p, BT, tiles, slices);
   g_colsum_rows = ((p.M + BT - 1) / BT) * (ks2 ? 4 : 2);  // per wave row and K group
   const dim3 grid(tiles, slices), block(ks2 ? 2 * V2_NT : V2_NT);
+  if constexpr (U && BT == 64 && (TA || !TB)) {
+    if ((TA && p.M < BT) || (!TB && p.N < BT)) {
+      if (ks2)
+        hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, 64, true, 2, true, true>), grid, block, 0, s, p);
+      else
+        hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, 64, true, 1, true, true>), grid, block, 0, s, p);
+      return hipGetLastError();
+    }
+  }
   if constexpr (U) {
     if (BT == 64 && ks2)
       hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, 64, true, 2, true>), grid, block, 0, s, p);
