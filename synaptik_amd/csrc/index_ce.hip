@@ -75,6 +75,15 @@ __global__ void __launch_bounds__(256) ce_rows_wave(CeArgs a) {
   const int64_t t = (int64_t)static_cast<const T*>(a.target)[r];
   const bool ignored = a.has_ignore && t == a.ignore;
   const bool in_range = t >= 0 && t < a.C;
+  if (ignored) {  // (uniform for the wave) no loss, a zero gradient: the row is not read
+    if (lane == 0) a.row_loss[r] = 0.0f;
+    if (a.grad != nullptr) {
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        if (lane + 64 * i < C) a.grad[r * a.C + lane + 64 * i] = 0.0f;
+    }
+    return;
+  }
   const int safe = (int)(t < 0 ? 0 : (t >= a.C ? a.C - 1 : t));
   const float xt = row[safe];
   float v[V];
@@ -97,9 +106,9 @@ __global__ void __launch_bounds__(256) ce_rows_wave(CeArgs a) {
   }
   const float sum = (float)wave_sum(s);
   if (lane == 0) {
-    if (!ignored && !in_range) atomicOr(a.status, (uint32_t)DEV_INDEX_OUT_OF_BOUNDS);
+    if (!in_range) atomicOr(a.status, (uint32_t)DEV_INDEX_OUT_OF_BOUNDS);
     const float lse = m + (float)log((double)sum);
-    a.row_loss[r] = !ignored && in_range ? lse - xt : 0.0f;
+    a.row_loss[r] = in_range ? lse - xt : 0.0f;
   }
   if (a.grad == nullptr) return;
   float* gr = a.grad + r * a.C;
@@ -107,7 +116,7 @@ __global__ void __launch_bounds__(256) ce_rows_wave(CeArgs a) {
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     const int c = lane + 64 * i;
-    if (c < C) gr[c] = ignored ? 0.0f : (v[i] / sum - (c == safe ? 1.0f : 0.0f)) * scale;
+    if (c < C) gr[c] = (v[i] / sum - (c == safe ? 1.0f : 0.0f)) * scale;
   }
 }
 
@@ -205,6 +214,12 @@ __global__ void __launch_bounds__(CE_STREAM_NT) ce_rows_stream(CeArgs a) {
     const int64_t t = (int64_t)static_cast<const T*>(a.target)[r];
     const bool ignored = a.has_ignore && t == a.ignore;
     const bool in_range = t >= 0 && t < a.C;
+    if (ignored) {  // as in ce_rows_block
+      if (threadIdx.x == 0) a.row_loss[r] = 0.0f;
+      if (a.grad != nullptr)
+        for (int64_t c = threadIdx.x; c < a.C; c += NT) a.grad[r * a.C + c] = 0.0f;
+      continue;
+    }
     const int64_t safe = t < 0 ? 0 : (t >= a.C ? a.C - 1 : t);
     const float xt = row[safe];
     float m = -INFINITY;
@@ -221,15 +236,15 @@ __global__ void __launch_bounds__(CE_STREAM_NT) ce_rows_stream(CeArgs a) {
     for (int64_t c = threadIdx.x; c < a.C; c += NT) s += (double)exp_rn(row[c] - m);
     const float sum = (float)block_sum<NT>(s, dl);
     if (threadIdx.x == 0) {
-      if (!ignored && !in_range) atomicOr(a.status, (uint32_t)DEV_INDEX_OUT_OF_BOUNDS);
+      if (!in_range) atomicOr(a.status, (uint32_t)DEV_INDEX_OUT_OF_BOUNDS);
       const float lse = m + (float)log((double)sum);
-      a.row_loss[r] = !ignored && in_range ? lse - xt : 0.0f;
+      a.row_loss[r] = in_range ? lse - xt : 0.0f;
     }
     if (a.grad == nullptr) continue;
     const float inv = 1.0f / sum;
     for (int64_t c = threadIdx.x; c < a.C; c += NT)
       a.grad[r * a.C + c] =
-          ignored ? 0.0f : (ce_quotient(exp_rn(row[c] - m), sum, inv) - (c == safe ? 1.0f : 0.0f)) * scale;
+          (ce_quotient(exp_rn(row[c] - m), sum, inv) - (c == safe ? 1.0f : 0.0f)) * scale;
   }
 }
 

@@ -79,3 +79,35 @@ def test_special_rows(ctx):
         assert np.array_equal(np.isnan(got), np.isnan(want))
         fin = ~np.isnan(want)
         np.testing.assert_allclose(got[fin], want[fin], rtol=1e-5, atol=1e-9)
+
+
+@pytest.mark.parametrize("R,C", [(70003, 3), (33000, 70), (1030, 1100), (9, 70001)])
+def test_mostly_ignored_rows(ctx, R, C):
+    """Ignored rows are not read: their logits are NaN here, their gradient is zero; the counts of
+    four parts of the rows, and a mean over more rows than one round of loads."""
+    print(f"[index_ce] ignored R={R} C={C}", flush=True)
+    rng = np.random.default_rng(R)
+    logits = rng.standard_normal((R, C)).astype(np.float32)
+    y = rng.integers(0, C, R)
+    skipped = rng.random(R) < 0.85
+    skipped[0] = False
+    y[skipped] = -7
+    read = logits.copy()
+    read[skipped] = np.nan
+    pb = ProgramBuilder()
+    sx, sy = pb.input(R * C), pb.input(R, "i64")
+    sl, sl2, sg = pb.output(1), pb.output(1), pb.output(R * C)
+    pb.index_ce(sx, sy, sl, R, C, grad=sg, ignore_index=-7)
+    pb.index_ce(sx, sy, sl2, R, C, ignore_index=-7)
+    loss, loss2, grad = run_program(ctx, pb, [read, y.astype(np.int64)], [sl, sl2, sg])
+    d = (logits - logits.max(1, keepdims=True)).astype(np.float64)
+    total = np.exp(d).sum(1)
+    rows = np.flatnonzero(~skipped)
+    exact = float(np.mean(np.log(total[rows]) - d[rows, y[rows]]))
+    # a row's loss is off by a few units of its largest term, about 2^-22 of the mean
+    assert abs(loss[0] - exact) <= 1e-6 * abs(exact) and loss2[0] == loss[0]
+    grad = grad.reshape(R, C)
+    assert not grad[skipped].any()
+    want = np.exp(d[rows]) / total[rows, None]
+    want[np.arange(len(rows)), y[rows]] -= 1.0
+    np.testing.assert_allclose(grad[rows], want / len(rows), rtol=2e-6, atol=2e-7 / len(rows))
