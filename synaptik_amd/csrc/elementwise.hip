@@ -339,8 +339,10 @@ __global__ void __launch_bounds__(256) colsum_pass1(const float* __restrict__ x,
 // 16-byte load per row (at any float), so a wave moves 1 KiB per row and a block covers 256
 // columns with 16 waves (rows r0 + w, r0 + w + 16, ..., four loads in flight each; a quarter of
 // colsum_pass1's blocks, so four times its waves). With 4-byte loads too few bytes are in flight:
-// [20000, 1001] 40.8 us on MI355X, 21.7 so.
-constexpr int CS_WAVES = 16;
+// [20000, 1001] 40.8 us on MI355X, 21.7 so. Up to CS_FEW_ROWS rows four waves do: the others
+// would only be launched and waited for ([8, 1000000] 27.3 us a call against 33.4).
+constexpr int64_t CS_FEW_ROWS = 32;
+template <int CS_WAVES>
 __global__ void __launch_bounds__(64 * CS_WAVES) colsum_pass1_v4(const float* __restrict__ x,
                                                                 double* part, int64_t R, int64_t N,
                                                                 int64_t ldx, int64_t rows) {
@@ -852,9 +854,12 @@ hipError_t launch_colsum(const float* x, float* out, int64_t R, int64_t N, int64
   const int64_t rows = colsum_rows_per_panel(R, N);
   const int64_t P = (R + rows - 1) / rows;
   if (P > 0) {
-    if (N >= 4 * CS_COLS) {
+    if (N > CS_COLS) {  // (64 columns fill colsum_pass1's lanes: [1000000, 33] 120 us, 144 in fours)
       dim3 g1((unsigned)((N + 4 * CS_COLS - 1) / (4 * CS_COLS)), (unsigned)P);
-      hipLaunchKernelGGL(colsum_pass1_v4, g1, dim3(64 * CS_WAVES), 0, s, x, partial, R, N, ldx, rows);
+      if (R <= CS_FEW_ROWS)
+        hipLaunchKernelGGL(colsum_pass1_v4<4>, g1, dim3(256), 0, s, x, partial, R, N, ldx, rows);
+      else
+        hipLaunchKernelGGL(colsum_pass1_v4<16>, g1, dim3(1024), 0, s, x, partial, R, N, ldx, rows);
     } else {
       dim3 g1((unsigned)((N + CS_COLS - 1) / CS_COLS), (unsigned)P);
       hipLaunchKernelGGL(colsum_pass1, g1, dim3(256), 0, s, x, partial, R, N, ldx, rows);

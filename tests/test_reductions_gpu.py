@@ -44,6 +44,13 @@ def test_row_reductions(ctx, C):
         np.testing.assert_allclose(got[fin], want[fin], rtol=tol, atol=0)
 
 
+@pytest.mark.parametrize("R,N", [(40000, 64), (40000, 65), (40001, 100), (33000, 255), (32, 300),
+                                 (33, 300), (1, 1000)])
+def test_column_sums_at_the_dispatch_edges(ctx, R, N):
+    """4-byte lanes up to 64 columns, four columns a lane beyond; four waves up to 32 rows."""
+    test_column_sums(ctx, R, N, 0)
+
+
 @pytest.mark.parametrize("R,N", [(70, 257), (1000, 1001), (17, 1023), (5000, 258), (3, 4099)])
 @pytest.mark.parametrize("pad", [0, 3])
 def test_column_sums(ctx, R, N, pad):
