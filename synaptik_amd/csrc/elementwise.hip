@@ -448,9 +448,13 @@ __global__ void __launch_bounds__(256) colsum_pass2(const double* part, float* o
 // Row reductions, binary64 accumulation for SUM/MEAN/LSE, one read of each row in aligned 16-byte
 // groups (rowvec.h), V of them a thread held in registers (LOG_SUM_EXP looks at them twice). Rows of
 // at most 2044 take one wave each: a workgroup a row spends its time in barriers and a single
-// load's latency. Wider rows take a workgroup of 256, rows beyond 8188 are read 4 bytes at a time
-// (twice for LOG_SUM_EXP). [20000, 1001] on MI355X, one workgroup a row with 4-byte loads before:
-// MAX 39, MEAN 22, LOG_SUM_EXP 58 us; now 14, 16 and 30.
+// load's latency. Wider rows take a workgroup of 256. From 8189 on SUM and MEAN read 4 bytes at a
+// time, eight loads in flight ([20000, 20000] 269 us a call, held by 1024 threads 363); MAX and
+// LOG_SUM_EXP, which look at a value twice or have more to do for it, are held by 512 and from
+// 16381 on by 1024 threads up to 32764, then read 4 bytes at a time (once more for LOG_SUM_EXP).
+// MI355X, one workgroup of 256 a row with 4-byte loads before: [20000, 1001] MAX 39, MEAN 22,
+// LOG_SUM_EXP 58 us, now 14, 16 and 30; LOG_SUM_EXP of [65536, 10000] 1465 us a call, now 843, of
+// [3000, 30000] 259, now 151, of [64, 100000] 159, now 92.
 constexpr int RR_NT = 256;
 
 __device__ __forceinline__ float row_lse(float m, float shift, double s) {
@@ -553,13 +557,14 @@ __global__ void __launch_bounds__(RR_NT) row_reduce_wave(const float* __restrict
   if (lane == 0) out[r] = result;
 }
 
-// One workgroup a row; V = 0: any width.
-template <int KIND, int V>
-__global__ void __launch_bounds__(RR_NT) row_reduce_block(const float* __restrict__ x, float* out,
-                                                          int64_t R, int64_t C) {
-  __shared__ double dl[RR_NT / 64];
-  __shared__ float fl[RR_NT / 64];
-  __shared__ int nl[RR_NT / 64];
+// One workgroup of NT threads a row; V = 0: any width.
+template <int NT, int KIND, int V>
+__global__ void __launch_bounds__(NT) row_reduce_block(const float* __restrict__ x, float* out,
+                                                       int64_t R, int64_t C) {
+  constexpr int NW = NT / 64;
+  __shared__ double dl[NW];
+  __shared__ float fl[NW];
+  __shared__ int nl[NW];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int64_t r = blockIdx.x; r < R; r += gridDim.x) {
     const float* row = x + r * C;
@@ -568,51 +573,59 @@ __global__ void __launch_bounds__(RR_NT) row_reduce_block(const float* __restric
       if constexpr (KIND < 2) {
         double s = 0.0;
 #pragma unroll 8
-        for (int64_t c = tid; c < C; c += RR_NT) s += (double)row[c];
-        s = block_sum<RR_NT>(s, dl);
+        for (int64_t c = tid; c < C; c += NT) s += (double)row[c];
+        s = block_sum<NT>(s, dl);
         if (tid == 0) out[r] = KIND == 1 ? (float)(s / (double)C) : (float)s;
       } else {
         float m = -INFINITY;
-        for (int64_t c = tid; c < C; c += RR_NT) m = java_max(m, row[c]);
-        m = block_max<RR_NT>(m, fl);
+        for (int64_t c = tid; c < C; c += NT) m = java_max(m, row[c]);
+        m = block_max<NT>(m, fl);
         if constexpr (KIND == 2) {
           if (tid == 0) out[r] = m;
         } else {
           const float shift = (m == INFINITY || m == -INFINITY) ? 0.0f : m;
           double s = 0.0;
-          for (int64_t c = tid; c < C; c += RR_NT) s += (double)exp_rn(row[c] - shift);
-          s = block_sum<RR_NT>(s, dl);
+          for (int64_t c = tid; c < C; c += NT) s += (double)exp_rn(row[c] - shift);
+          s = block_sum<NT>(s, dl);
           if (tid == 0) out[r] = row_lse(m, shift, s);
         }
       }
     } else {
       const RowGroups view(row, (int)C);
       RowPart<V> part;
-      part.template load<RR_NT>(view, row, tid, KIND >= 2 ? -INFINITY : 0.0f);
+      part.template load<NT>(view, row, tid, KIND >= 2 ? -INFINITY : 0.0f);
       if constexpr (KIND < 2) {
-        const double s = block_sum<RR_NT>(part.sum(), dl);
+        const double s = block_sum<NT>(part.sum(), dl);
         if (tid == 0) out[r] = KIND == 1 ? (float)(s / (double)C) : (float)s;
       } else {
         int nan;
         float m = wave_fmax(part.maximum(nan));
         nan = __any(nan);
+        auto any = [&]() {
+          int a = nl[0];
+#pragma unroll
+          for (int i = 1; i < NW; ++i) a |= nl[i];
+          return a;
+        };
         if (lane == 0) { fl[w] = m; nl[w] = nan; }
         __syncthreads();
-        m = fmaxf(fmaxf(fl[0], fl[1]), fmaxf(fl[2], fl[3]));
-        if (nl[0] | nl[1] | nl[2] | nl[3]) {
+        m = fl[0];
+#pragma unroll
+        for (int i = 1; i < NW; ++i) m = fmaxf(m, fl[i]);
+        if (any()) {
           m = NAN;
         } else if (m == 0.0f) {  // the same for the whole workgroup
           const int z = __any(part.positive_zero());
           __syncthreads();
           if (lane == 0) nl[w] = z;
           __syncthreads();
-          m = (nl[0] | nl[1] | nl[2] | nl[3]) ? 0.0f : -0.0f;
+          m = any() ? 0.0f : -0.0f;
         }
         if constexpr (KIND == 2) {
           if (tid == 0) out[r] = m;
         } else {
           const float shift = (m == INFINITY || m == -INFINITY) ? 0.0f : m;
-          const double s = block_sum<RR_NT>(part.sum_exp(shift), dl);
+          const double s = block_sum<NT>(part.sum_exp(shift), dl);
           if (tid == 0) out[r] = row_lse(m, shift, s);
         }
       }
@@ -628,9 +641,13 @@ void launch_row_kind(const float* x, float* out, int64_t R, int64_t C, hipStream
   else if (C <= 64 * 4 * 2 - 4) hipLaunchKernelGGL((row_reduce_wave<KIND, 2>), quads, nt, 0, s, x, out, R, C);
   else if (C <= 64 * 4 * 4 - 4) hipLaunchKernelGGL((row_reduce_wave<KIND, 4>), quads, nt, 0, s, x, out, R, C);
   else if (C <= 64 * 4 * 8 - 4) hipLaunchKernelGGL((row_reduce_wave<KIND, 8>), quads, nt, 0, s, x, out, R, C);
-  else if (C <= RR_NT * 4 * 4 - 4) hipLaunchKernelGGL((row_reduce_block<KIND, 4>), rows, nt, 0, s, x, out, R, C);
-  else if (C <= RR_NT * 4 * 8 - 4) hipLaunchKernelGGL((row_reduce_block<KIND, 8>), rows, nt, 0, s, x, out, R, C);
-  else hipLaunchKernelGGL((row_reduce_block<KIND, 0>), rows, nt, 0, s, x, out, R, C);
+  else if (C <= 256 * 4 * 4 - 4) hipLaunchKernelGGL((row_reduce_block<256, KIND, 4>), rows, nt, 0, s, x, out, R, C);
+  else if (C <= 256 * 4 * 8 - 4) hipLaunchKernelGGL((row_reduce_block<256, KIND, 8>), rows, nt, 0, s, x, out, R, C);
+  else if constexpr (KIND < 2)
+    hipLaunchKernelGGL((row_reduce_block<256, KIND, 0>), rows, nt, 0, s, x, out, R, C);
+  else if (C <= 512 * 4 * 8 - 4) hipLaunchKernelGGL((row_reduce_block<512, KIND, 8>), rows, dim3(512), 0, s, x, out, R, C);
+  else if (C <= 1024 * 4 * 8 - 4) hipLaunchKernelGGL((row_reduce_block<1024, KIND, 8>), rows, dim3(1024), 0, s, x, out, R, C);
+  else hipLaunchKernelGGL((row_reduce_block<512, KIND, 0>), rows, dim3(512), 0, s, x, out, R, C);
 }
 
 // Whole-tensor reductions in two deterministic passes.

@@ -1,6 +1,6 @@
 """Row, column and whole-tensor reductions at the edges of their kernels' widths: one wave a row up
-to 2044 columns, one workgroup up to 8188, re-read beyond; rows whose start is not 16-byte aligned;
-column sums whose last lane holds one to three columns."""
+to 2044 columns, one workgroup of 256 up to 8188, of 512 up to 16380 and of 1024 up to 32764, re-read
+beyond; rows whose start is not 16-byte aligned; column sums whose last lane holds one to three columns."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,7 @@ from tests.gpu_helpers import run_program
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("C", [1, 3, 65, 252, 253, 508, 509, 1001, 1020, 1021, 2044, 2045, 4092, 4093, 8188, 8189, 20003])
+@pytest.mark.parametrize("C", [1, 3, 65, 252, 253, 508, 509, 1001, 1020, 1021, 2044, 2045, 4092, 4093, 8188, 8189, 16380, 16381, 20003, 32764, 32767, 70001])
 def test_row_reductions(ctx, C):
     print(f"[row_reduce] C={C}", flush=True)
     R = 9
