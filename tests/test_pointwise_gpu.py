@@ -1,6 +1,6 @@
 """The chain interpreter at the places where its index arithmetic can go wrong: widths around a
-group of four, groups that span rows, the last partial group, more groups than one round of
-threads takes, and chains of both broadcast kinds, against numpy in the same binary32 operations."""
+group of four, groups that span rows, the last partial group, and chains of both broadcast kinds,
+against numpy in the same binary32 operations. (More than one round of the grid: test_many_rows_gpu.)"""
 import numpy as np
 import pytest
 
@@ -34,7 +34,7 @@ def test_broadcast_chain(ctx, R, C):
 
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 1023, 2560 * 1024 + 3, 3 * 2560 * 1024 + 1])
 def test_long_chain(ctx, n):
-    """No broadcast: several rounds of the grid, each with its inputs loaded ahead."""
+    """No broadcast: the last group and the last workgroup partly filled."""
     rng = np.random.default_rng(n)
     x, y = (rng.standard_normal(n).astype(np.float32) for _ in range(2))
     pb = ProgramBuilder()
