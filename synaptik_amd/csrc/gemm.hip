@@ -185,11 +185,11 @@ __global__ void __launch_bounds__(256) gemm_splitk_reduce4(GemmParams p, int spl
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 
-hipError_t launch_tiles(const GemmParams& p, bool va, bool vb, bool split, hipStream_t s) {
-  if (!p.transA && !p.transB) return launch_layout<false, false>(p, va, vb, split, s);
-  if (!p.transA && p.transB) return launch_layout<false, true>(p, va, vb, split, s);
-  if (p.transA && !p.transB) return launch_layout<true, false>(p, va, vb, split, s);
-  return launch_layout<true, true>(p, va, vb, split, s);
+hipError_t launch_tiles(const GemmParams& p, bool va, bool vb, hipStream_t s) {
+  if (!p.transA && !p.transB) return launch_layout<false, false>(p, va, vb, s);
+  if (!p.transA && p.transB) return launch_layout<false, true>(p, va, vb, s);
+  if (p.transA && !p.transB) return launch_layout<true, false>(p, va, vb, s);
+  return launch_layout<true, true>(p, va, vb, s);
 }
 
 }  // namespace
@@ -320,7 +320,7 @@ hipError_t launch_gemm_core(const GemmParams& in, float* workspace, hipStream_t 
     p.partial = workspace;
     bool va, vb;
     vector_operands(p, va, vb);
-    hipError_t e = launch_tiles(p, va, vb, true, s);
+    hipError_t e = launch_tiles(p, va, vb, s);
     if (e != hipSuccess) return e;
     return launch_splitk_finish(p, slices, s);
   }
@@ -332,7 +332,7 @@ hipError_t launch_gemm_core(const GemmParams& in, float* workspace, hipStream_t 
   }
   bool va, vb;
   vector_operands(p, va, vb);
-  return launch_tiles(p, va, vb, false, s);
+  return launch_tiles(p, va, vb, s);
 }
 
 hipError_t launch_splitk_finish(const GemmParams& p, int slices, hipStream_t s) {

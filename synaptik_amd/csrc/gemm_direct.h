@@ -1,5 +1,6 @@
 // fp32 MFMA GEMM straight from memory to registers, for gfx950: the problems with too few tiles
-// for the direct-to-LDS kernel (gemm_v2.h), and the few whose operands it cannot address.
+// for the direct-to-LDS kernel (gemm_v2.h), and the few with more that it does not take
+// (direct_wide).
 //
 // Such a problem is bound by latency: a 128 x 1024 x 512 product is 1 us of matrix work. A wave
 // owns a WT x WT tile (WT = 16 NB) as NB x NB blocks of v_mfma_f32_16x16x4_f32 and loads its operand
@@ -78,16 +79,10 @@ struct DirectOperand {
       for (int s = 0; s < 4; ++s) {
         const float* src = p[0] + step + s * ld;
         if (!edge) {
-          if constexpr (NB == 4) {
-            const float4u v = *reinterpret_cast<const float4u*>(src + row0);
-#pragma unroll
-            for (int b = 0; b < NB; ++b) f[b][s] = v[b];
-          } else {
-            static_assert(NB == 2, "two or four blocks");
-            const float2u v = *reinterpret_cast<const float2u*>(src + row0);
-            f[0][s] = v[0];
-            f[1][s] = v[1];
-          }
+          static_assert(NB == 2, "two adjacent rows a lane");
+          const float2u v = *reinterpret_cast<const float2u*>(src + row0);
+          f[0][s] = v[0];
+          f[1][s] = v[1];
         } else {
 #pragma unroll
           for (int b = 0; b < NB; ++b) f[b][s] = src[min(row0 + b, rows - 1)];
@@ -115,7 +110,7 @@ template <int NB, int MW, int NW, int KW>
 struct DirectCfg {
   static constexpr int WT = 16 * NB, TM = WT * MW, TN = WT * NW;
   static constexpr int NT = 64 * MW * NW * KW;
-  static constexpr int D = NB == 4 ? 2 : 4;        // steps in flight
+  static constexpr int D = 4;                      // steps in flight
   static constexpr int CH = TN / 4;                // 16-byte chunks per tile row
   static constexpr int SW = (CH < 16 ? CH : 16) - 1;
   static constexpr int RP = NT / CH;               // rows per epilogue pass
@@ -240,13 +235,8 @@ gemm_direct(GemmParams p) {
         static_for<4>([&](auto r) {
           constexpr int I = decltype(i)::value, R = decltype(r)::value;
           float* dst = at(KA ? 16 * I + 4 * g + R : NB * (4 * g + R) + I, NB * l16);
-          if constexpr (NB == 4) {
-            *reinterpret_cast<floatx4*>(dst) =
-                floatx4{acc[I][0][R], acc[I][1][R], acc[I][2][R], acc[I][3][R]};
-          } else {
-            typedef float floatx2 __attribute__((ext_vector_type(2)));
-            *reinterpret_cast<floatx2*>(dst) = floatx2{acc[I][0][R], acc[I][1][R]};
-          }
+          typedef float floatx2 __attribute__((ext_vector_type(2)));
+          *reinterpret_cast<floatx2*>(dst) = floatx2{acc[I][0][R], acc[I][1][R]};
         });
       });
     }
@@ -424,8 +414,11 @@ hipError_t launch_direct_cfg(const GemmParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// 64x64 tiles once they give every CU a workgroup (2000x300x200 NT 10.7 us against 11.0 with
-// 32x32 tiles, 1024x1024x784 20.6 against 29.7), 32x32 below (500x509x1021 12.2 against 25.2).
+// 64x64 tiles once they give every CU a workgroup, 32x32 below. Problems with that many tiles come
+// here where gemm_v2.h refuses them: unaligned products of 17 to 32 rows or columns (whole calls:
+// 200001x25x33 NN 39.3 us on 64x64 tiles, 48.9 on 32x32; 200001x25x200 78.6 and 79.5; TN
+// 200001x25x33 52.9 and 62.1; fewer tiles 8200x19x300 NN 22.0 and 19.9), or of 33 to 63 with little K
+// (30001x63x33 NN 19.6 and 25.0); leading dimensions beyond its offsets; K < 4.
 inline bool direct_wide(const GemmParams& p) {
   const int64_t slices = p.kchunk > 0 ? (p.K + p.kchunk - 1) / p.kchunk : 1;
   return ((p.M + 63) / 64) * ((p.N + 63) / 64) * slices >= 256;

@@ -30,13 +30,13 @@ namespace shk {
 extern thread_local int64_t g_colsum_rows;
 
 // Launches an MFMA kernel for one operand layout (instantiated per layout).
-//   va / vb: the A / B operand allows float4 loads; split: p.kchunk > 0 (split-K slices).
+//   va / vb: the A / B operand allows aligned float4 loads; p.kchunk > 0: split-K slices.
 template <bool TA, bool TB>
-hipError_t launch_layout(const GemmParams& p, bool va, bool vb, bool split, hipStream_t s);
-extern template hipError_t launch_layout<false, false>(const GemmParams&, bool, bool, bool, hipStream_t);
-extern template hipError_t launch_layout<false, true>(const GemmParams&, bool, bool, bool, hipStream_t);
-extern template hipError_t launch_layout<true, false>(const GemmParams&, bool, bool, bool, hipStream_t);
-extern template hipError_t launch_layout<true, true>(const GemmParams&, bool, bool, bool, hipStream_t);
+hipError_t launch_layout(const GemmParams& p, bool va, bool vb, hipStream_t s);
+extern template hipError_t launch_layout<false, false>(const GemmParams&, bool, bool, hipStream_t);
+extern template hipError_t launch_layout<false, true>(const GemmParams&, bool, bool, hipStream_t);
+extern template hipError_t launch_layout<true, false>(const GemmParams&, bool, bool, hipStream_t);
+extern template hipError_t launch_layout<true, true>(const GemmParams&, bool, bool, hipStream_t);
 
 namespace {
 

@@ -57,7 +57,7 @@ constexpr int V2_GROUP = 4, V2_GROUP64 = 2;
 //     tile stays where it is: its last chunk at each k takes in up to three floats of the row after
 //     (they reach only results that are not stored), and at the last k it is loaded float by float;
 //   * the chunk of a K-contiguous row that K cuts is loaded float by float (once per tile).
-template <int BT, bool U>
+template <int BT>
 struct V2Cfg {
   static constexpr int NB = BT / 32;      // 16x16 blocks per wave and dimension
   static constexpr int WT = BT / 2;       // wave tile edge
@@ -75,7 +75,7 @@ struct V2Cfg {
 // CUT: an M/N-contiguous operand of less than a tile (see U above).
 template <bool KMAJ, int BT, bool TAIL, bool U, bool CUT>
 struct V2Loader {
-  using Cfg = V2Cfg<BT, U>;
+  using Cfg = V2Cfg<BT>;
   uint32_t voff[Cfg::NI];
   int vrow[Cfg::NI], vk[Cfg::NI];  // first row (M/N) and first k of the chunk in the tile
   uint32_t wdst;                   // this wave's byte offset inside a stage (wave-uniform)
@@ -154,7 +154,7 @@ struct V2Loader {
 // the accumulators back through the same interleave (v2_row / v2_col).
 template <bool KMAJ, int BT>
 struct V2Frag {
-  static constexpr int NB = V2Cfg<BT, false>::NB;
+  static constexpr int NB = V2Cfg<BT>::NB;
   static constexpr int ITEMS = KMAJ ? NB : 4;  // fragment reads per half
   floatx4 f[NB];
   template <int H, int T>
@@ -257,7 +257,7 @@ template <bool KA, bool KB, int BT, bool TAIL, int KS, bool U = false, bool CUT 
 __global__ void __launch_bounds__(V2_NT * KS) __attribute__((amdgpu_waves_per_eu(2)))
 gemm_f32_v2(GemmParams p) {
   static_assert(!U || TAIL, "operands of any alignment have edges");
-  using Cfg = V2Cfg<BT, U>;
+  using Cfg = V2Cfg<BT>;
   constexpr int NB = Cfg::NB, WT = Cfg::WT, TILEF = Cfg::TILEF, NI = Cfg::NI, NG = Cfg::NG;
   __shared__ __attribute__((aligned(16))) float As0g[KS * TILEF];
   __shared__ __attribute__((aligned(16))) float Bs0g[KS * TILEF];
@@ -782,7 +782,8 @@ constexpr int64_t V2_MAX_TILES = (1LL << 32) / V2_NT;
 //     rows or columns from 512 tiles on, from 256 with K > 64 (30001x63x1021 NN 53 here, 96 and 106
 //     on gemm_direct's 32x32 and 64x64 tiles, TN 53 against 109 and 121; 30001x63x33 NN 20.1 against
 //     25.0 and 19.6). With fewer only TN, whose fragments gemm_direct reads 8 bytes at a time, from
-//     K = 128 on (17x30001x509 TN 38.9 against 52.6; NN 30001x17x509 40.7 against 34.6).
+//     K = 192 on (17x30001x509 TN 38.9 against 52.6, 30001x25x200 27.7 against 29.4, x130 24.3 against
+//     23.2; NN 30001x17x509 40.7 against 34.6).
 // TAIL variants run when M, N or K (or the slice) is not a whole number of tiles.
 inline int v2_choose(const GemmParams& p, bool aligned) {
   if (p.K < 4 || (p.kchunk > 0 && (p.kchunk % V2_BK != 0 || p.partial == nullptr))) return 0;
@@ -793,7 +794,7 @@ inline int v2_choose(const GemmParams& p, bool aligned) {
   auto enough = [&](int64_t extent, int bt) {
     if (aligned || extent >= bt) return true;
     if (bt != 64 || p.kchunk > 0 || t64 < 256) return false;
-    return extent > 32 ? p.K > 64 || t64 >= 512 : p.transA && !p.transB && p.K >= 128;
+    return extent > 32 ? p.K > 64 || t64 >= 512 : p.transA && !p.transB && p.K >= 192;
   };
   auto fits = [&](int bt) {
     return (!p.transA || enough(p.M, bt)) && (p.transB || enough(p.N, bt)) &&

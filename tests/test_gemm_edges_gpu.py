@@ -52,7 +52,7 @@ def test_exact_products(ctx, M, N, K, ta, tb, pad):
 
 # M/N-contiguous operands of less than a 64-wide tile, many tiles along the other extent: LDS tiles
 # whose chunks run past the operand's row, 64x64 register tiles (the last three), by layout and K
-NARROW = [(33, 17000, 67), (17000, 63, 97), (61, 16500, 520), (20, 16500, 130), (33000, 33, 33),
+NARROW = [(33, 17000, 67), (17000, 63, 97), (61, 16500, 520), (20, 16500, 200), (33000, 33, 33),
           (16500, 17, 19), (31, 16500, 19), (16385, 32, 127)]
 
 
