@@ -28,9 +28,8 @@ namespace {
 
 constexpr int SK_J = 16;  // largest narrow extent
 
-__device__ __forceinline__ bool epilogue_store(const GemmParams& p, const UpdateCtx& uc,
-                                               int64_t row, int64_t col, float v) {
-  if (p.upd.pn != nullptr) return update_scalar(p.upd, uc, row * p.N + col, v);
+__device__ __forceinline__ void epilogue_store(const GemmParams& p, int64_t row, int64_t col,
+                                               float v) {
   if (p.mode == 0) {
     if (p.bias != nullptr) v = v + p.bias[col];
     v = apply_act(p.act, v);
@@ -40,6 +39,12 @@ __device__ __forceinline__ bool epilogue_store(const GemmParams& p, const Update
   float* dst = p.C + row * p.ldc + col;
   if (p.accumulate) v = *dst + v;
   *dst = v;
+}
+// The same, or the staged update: true unless one of its checks failed.
+__device__ __forceinline__ bool epilogue_or_update(const GemmParams& p, const UpdateCtx& uc,
+                                                   int64_t row, int64_t col, float v) {
+  if (p.upd.pn != nullptr) return update_scalar(p.upd, uc, row * p.N + col, v);
+  epilogue_store(p, row, col, v);
   return true;
 }
 
@@ -96,16 +101,20 @@ constexpr int64_t SMALL_K_NARROW_N = 128;
 // per-element work (a binary64 tanh, say) four times the waves instead of a serial loop.
 template <int CPL>
 constexpr int small_k_rb() { return CPL == 1 ? 1 : SK_RB; }
-template <int KB, int CPL>
+// UPD: the staged update, in kernels of its own: with the activations in the same kernel its
+// scalar values are spilled into vector registers and read back for every element (Adam on
+// 11136x4330x11 NN 612 us a call on MI355X, 575 so; 1024x1024x10 TN 33.9, 29.2 so).
+template <int KB, int CPL, bool UPD>
 __global__ void __launch_bounds__(256) gemm_small_k(GemmParams p, int vec_b, int vec_io) {
   constexpr int RB = small_k_rb<CPL>();
   __shared__ double csum[4][64 * CPL];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t c0 = ((int64_t)blockIdx.x * 64 + lane) * CPL;
-  bool ok;
-  const UpdateCtx uc = begin_update(p, ok);
+  bool ok = true;
+  UpdateCtx uc{};
+  if constexpr (UPD) uc = begin_update(p, ok);
   const int K = (int)p.K;
-  const bool want_sum = p.colsum_partial != nullptr;
+  const bool want_sum = !UPD && p.colsum_partial != nullptr;
   double cs[CPL];
 #pragma unroll
   for (int c = 0; c < CPL; ++c) cs[c] = 0.0;
@@ -115,7 +124,7 @@ __global__ void __launch_bounds__(256) gemm_small_k(GemmParams p, int vec_b, int
   {
     float b[KB][CPL];
     const bool full = c0 + 3 < p.N;
-    const bool v4 = CPL == 4 && vec_io && full;
+    const bool v4 = !UPD && CPL == 4 && vec_io && full;
 #pragma unroll
     for (int k = 0; k < KB; ++k) {
       const int64_t kk = k < K ? k : K - 1;
@@ -180,7 +189,8 @@ __global__ void __launch_bounds__(256) gemm_small_k(GemmParams p, int vec_b, int
 #pragma unroll
           for (int c = 0; c < CPL; ++c) {
             if (c0 + c < p.N) {
-              ok &= epilogue_store(p, uc, r, c0 + c, acc[c]);
+              if constexpr (UPD) ok &= update_scalar(p.upd, uc, r * p.N + c0 + c, acc[c]);
+              else epilogue_store(p, r, c0 + c, acc[c]);
               if (want_sum) cs[c] += (double)p.C[r * p.ldc + c0 + c];
             }
           }
@@ -198,7 +208,7 @@ __global__ void __launch_bounds__(256) gemm_small_k(GemmParams p, int vec_b, int
           ((csum[0][threadIdx.x] + csum[1][threadIdx.x]) + csum[2][threadIdx.x]) +
           csum[3][threadIdx.x];
   }
-  if (p.upd.pn != nullptr) update_flag(p.upd, uc, ok);
+  if constexpr (UPD) update_flag(p.upd, uc, ok);
 }
 
 // ---- row dot: D[r, j] = sum_k X[r*ldx + k] * Y(j, k), Y(j, k) = Y[j*ysj + k*ysk] ----
@@ -272,7 +282,7 @@ __global__ void __launch_bounds__(256) gemm_row_dot(GemmParams p, RowDot d) {
     for (int off = 32 >> LG; off >= 1; off >>= 1) acc[0] += __shfl_xor(acc[0], off, 64);
     const int j = lane >> (6 - LG);
     if ((lane & ((64 >> LG) - 1)) == 0 && j < d.J)
-      ok &= d.swap ? epilogue_store(p, uc, j, r, acc[0]) : epilogue_store(p, uc, r, j, acc[0]);
+      ok &= d.swap ? epilogue_or_update(p, uc, j, r, acc[0]) : epilogue_or_update(p, uc, r, j, acc[0]);
   }
   if (p.upd.pn != nullptr) update_flag(p.upd, uc, ok);
 }
@@ -402,12 +412,16 @@ template <int KB>
 struct SmallK {
   static hipError_t run(const GemmParams& p, int vec_b, int vec_io, hipStream_t s) {
     const int64_t y = small_k_row_blocks(p.M, p.N);
-    if (p.N <= SMALL_K_NARROW_N)
-      hipLaunchKernelGGL((gemm_small_k<KB, 1>), dim3((unsigned)((p.N + 63) / 64), (unsigned)y),
-                         dim3(256), 0, s, p, vec_b, vec_io);
+    const dim3 narrow((unsigned)((p.N + 63) / 64), (unsigned)y), wide((unsigned)((p.N + 255) / 256), (unsigned)y);
+    const bool upd = p.upd.pn != nullptr;
+    if (p.N <= SMALL_K_NARROW_N && upd)
+      hipLaunchKernelGGL((gemm_small_k<KB, 1, true>), narrow, dim3(256), 0, s, p, vec_b, vec_io);
+    else if (p.N <= SMALL_K_NARROW_N)
+      hipLaunchKernelGGL((gemm_small_k<KB, 1, false>), narrow, dim3(256), 0, s, p, vec_b, vec_io);
+    else if (upd)
+      hipLaunchKernelGGL((gemm_small_k<KB, 4, true>), wide, dim3(256), 0, s, p, vec_b, vec_io);
     else
-      hipLaunchKernelGGL((gemm_small_k<KB, 4>), dim3((unsigned)((p.N + 255) / 256), (unsigned)y),
-                         dim3(256), 0, s, p, vec_b, vec_io);
+      hipLaunchKernelGGL((gemm_small_k<KB, 4, false>), wide, dim3(256), 0, s, p, vec_b, vec_io);
     g_colsum_rows = y;
     return hipGetLastError();
   }
