@@ -15,6 +15,7 @@
 // Java Math.max (NaN wins, +0.0 beats -0.0).
 #include "common.h"
 #include "kernels.h"
+#include "pw_divide.h"
 #include "rowvec.h"
 #include <algorithm>
 #include <type_traits>
@@ -112,31 +113,15 @@ __global__ void __launch_bounds__(256) pw_single_kernel(const float* x,
   }
 }
 
-// Division of element ordinals below 2^32 by the row width C (Granlund and Montgomery, "Division
-// by invariant integers using multiplication", 1994): with l = ceil(log2 C) and
-// mul = floor(2^32 (2^l - C) / C) + 1, t = high half of mul n and n / C = (t + (n - t) / 2) >> (l - 1).
-struct PwDivide {
-  uint32_t mul, shift;
-  int narrow;  // every ordinal fits 32 bits and C > 1
-};
-PwDivide pw_divide(int64_t n, int64_t C) {
-  PwDivide d{0, 0, 0};
-  if (C <= 1 || n > 0xffffffffll) return d;
-  int l = 0;
-  while ((1ll << l) < C) ++l;
-  d.mul = (uint32_t)((((unsigned __int128)1 << 32) * (uint64_t)((1ll << l) - C)) / (uint64_t)C + 1);
-  d.shift = (uint32_t)(l - 1);
-  d.narrow = 1;
-  return d;
-}
-
 // The interpreter. A thread handles one group of four elements, whose register k lives in LDS at
 // regs[k * PW_NT + t]: any register index is just an address (no dynamically indexed VGPR array, no
 // scratch) and each operand access is one 128-bit LDS access per lane. A launch takes only as many
 // registers as its chain uses.
 //
 // What bounds it is the instructions around the arithmetic -- decoding, branching on the operation
-// and on each input's kind -- and how many waves share them: seven a SIMD. An ordinal is divided
+// and on each input's kind -- and how many waves share them: seven a SIMD for chains that name up
+// to five registers; six and five for six and for seven or eight, whose workgroups take 24 to 32 KB
+// of a CU's 160 KB of LDS. An ordinal is divided
 // once, by multiplication; a broadcast operand within one row is one vector load; an instruction
 // is read as words (read as bytes it would come through vector memory: scalar loads have none), the
 // next one's ahead of time. Before: a 64-bit division and four loads for each broadcast operand,
@@ -199,8 +184,8 @@ pointwise_kernel(PwArgs a) {
         row = e0 / C;
         col = e0 - row * C;
       } else {
-        const uint32_t e = (uint32_t)e0, h = __umulhi(a.div.mul, e);
-        row = (h + ((e - h) >> 1)) >> a.div.shift;
+        const uint32_t e = (uint32_t)e0;
+        row = pw_quotient(a.div.mul, a.div.shift, e);
         col = e - row * C;
       }
     }
