@@ -5,15 +5,20 @@
 //   -inf (log-softmax); a row containing -inf (and no NaN) is evaluated unshifted (shift 0);
 //   addends are (float)exp((double)(x - shift)); the result is (float)exp(shift)/sum or
 //   shift - (float)log(sum). The GPU forms the addends with exp_f32 (fexp.h), which returns
-//   that binary32 value or one of its neighbours (at most 1 ulp away; 0.46% of arguments), and
-//   rows held in registers multiply by a once-rounded reciprocal of the sum.
+//   that binary32 value or one of its neighbours (at most 1 ulp away; 0.46% of arguments), in its
+//   range, and as the reference does elsewhere.
 //   The reference sums addends with Kahan compensation in binary32 (error within about
-//   2 ulp of the exact sum). Register-held rows sum each lane's 4V binary32 addends pairwise in
-//   binary32 (positive addends: error within log2(4V) ulp), combine the lanes in binary64
-//   through a fixed tree and round once; streamed rows sum in binary64 throughout. Both sums are
-//   within a few binary32 ulps of the exact sum (reduction-order difference).
-// One 256-thread workgroup owns one row; rows up to 4096 wide are held in registers
-// (one HBM read and one write per element), wider rows are streamed three times.
+//   2 ulp of the exact sum). All forms here round a sum once that is within a few binary32 ulps of
+//   the exact one (reduction-order difference):
+//   softmax_fwd_regs    16-byte aligned rows of 509 to 4096: one workgroup of 256 a row, held in
+//                       registers. Each lane's 4V addends are summed pairwise in binary32 (positive
+//                       addends: error within log2(4V) ulp), the lanes in binary64 through a fixed
+//                       tree; the row is multiplied by a once-rounded reciprocal of the sum.
+//   softmax_fwd_rows    other rows up to 32764 (aligned ones up to 32768): one wave or one workgroup
+//                       of 256 to 1024 a row, held in registers, summed in binary64; the quotient is
+//                       the correctly rounded one.
+//   softmax_fwd_stream  wider rows: one workgroup of 256 a row, read three times, summed in binary64
+//                       and divided.
 #include "common.h"
 #include "fexp.h"
 #include "kernels.h"
