@@ -403,11 +403,32 @@ __global__ void __launch_bounds__(1024) colsum_small(const float* __restrict__ x
     out[col] = v;
   }
 }
-// Column sums, pass 2: block x finishes 64 columns; wave w adds partial rows w, w + 4, ... in
-// two interleaved chains (independent loads in flight), then the chains and the four waves are
+// Many partial rows are folded first: block (x, y) adds rows y * chunk .. of 64 columns into the
+// first of them (in the order rows w, w + 4, ... of wave w, then the waves), eight loads in flight.
+// A single block of pass 2 per 64 columns takes 67 us for the 1876 rows that the bias gradient of
+// 30001 rows leaves on MI355X; folded, both launches take 9.5.
+constexpr int64_t CS_FOLD_ROWS = 256, CS_FOLD_CHUNK = 64;
+__global__ void __launch_bounds__(256) colsum_fold(double* part, int64_t P, int64_t N) {
+  __shared__ double lds[4][CS_COLS];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t col = (int64_t)blockIdx.x * CS_COLS + lane;
+  const int64_t r0 = (int64_t)blockIdx.y * CS_FOLD_CHUNK, rend = min(P, r0 + CS_FOLD_CHUNK);
+  double s = 0.0;
+  if (col < N) {
+#pragma unroll 8
+    for (int64_t i = r0 + w; i < rend; i += 4) s += part[i * N + col];
+  }
+  lds[w][lane] = s;
+  __syncthreads();  // (the block has read its rows)
+  if (w == 0 && col < N)
+    part[r0 * N + col] = ((lds[0][lane] + lds[1][lane]) + lds[2][lane]) + lds[3][lane];
+}
+// Column sums, pass 2: block x finishes 64 columns of P partial rows `step` apart; wave w adds
+// partial rows w, w + 4, ... in two interleaved chains (independent loads in flight), then the chains and the four waves are
 // combined in a fixed order, so results are run-to-run identical.
 __global__ void __launch_bounds__(256) colsum_pass2(const double* part, float* out, int64_t P,
-                                                    int64_t N, double divisor, int accumulate) {
+                                                    int64_t N, int64_t step, double divisor,
+                                                    int accumulate) {
   __shared__ double lds[4][CS_COLS];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t col = (int64_t)blockIdx.x * CS_COLS + lane;
@@ -415,10 +436,10 @@ __global__ void __launch_bounds__(256) colsum_pass2(const double* part, float* o
   if (col < N) {
     int64_t i = w;
     for (; i + 4 < P; i += 8) {
-      s0 += part[i * N + col];
-      s1 += part[(i + 4) * N + col];
+      s0 += part[i * step + col];
+      s1 += part[(i + 4) * step + col];
     }
-    if (i < P) s0 += part[i * N + col];
+    if (i < P) s0 += part[i * step + col];
   }
   lds[w][lane] = s0 + s1;
   __syncthreads();
@@ -868,15 +889,24 @@ hipError_t launch_colsum(const float* x, float* out, int64_t R, int64_t N, int64
     }
   }
   hipLaunchKernelGGL(colsum_pass2, dim3((unsigned)((N + CS_COLS - 1) / CS_COLS)), dim3(256), 0, s,
-                     partial, out, P, N, divisor, accumulate);
+                     partial, out, P, N, N, divisor, accumulate);
   return hipGetLastError();
 }
 
-hipError_t launch_colsum_finish(const double* partial, float* out, int64_t P, int64_t N,
+hipError_t launch_colsum_finish(double* partial, float* out, int64_t P, int64_t N,
                                 hipStream_t s) {
   if (N <= 0) return hipSuccess;
-  hipLaunchKernelGGL(colsum_pass2, dim3((unsigned)((N + CS_COLS - 1) / CS_COLS)), dim3(256), 0, s,
-                     partial, out, P, N, 1.0, 0);
+  const unsigned x = (unsigned)((N + CS_COLS - 1) / CS_COLS);
+  int64_t step = N;
+  // a fold's workgroups beyond the grid's second dimension: one pass reads them all, as it did
+  const int64_t chunks = (P + CS_FOLD_CHUNK - 1) / CS_FOLD_CHUNK;
+  if (P > CS_FOLD_ROWS && chunks < 65536) {
+    hipLaunchKernelGGL(colsum_fold, dim3(x, (unsigned)chunks), dim3(256), 0, s, partial, P, N);
+    P = chunks;
+    step = CS_FOLD_CHUNK * N;
+  }
+  hipLaunchKernelGGL(colsum_pass2, dim3(x), dim3(256), 0, s, (const double*)partial, out, P, N, step,
+                     1.0, 0);
   return hipGetLastError();
 }
 

@@ -74,7 +74,7 @@ struct GemmParams {
 hipError_t launch_gemm(const GemmParams& p, float* workspace, hipStream_t s);
 int64_t gemm_workspace_floats(int64_t M, int64_t N, int64_t K, bool colsum = false);
 // Finishes a column sum from P partial rows (binary64, fixed order) into out[N].
-hipError_t launch_colsum_finish(const double* partial, float* out, int64_t P, int64_t N,
+hipError_t launch_colsum_finish(double* partial, float* out, int64_t P, int64_t N,
                                 hipStream_t s);
 
 // Column sums of X[R,N] (row stride ldx) into out[N]; out = (float)(sum * scale_num / scale_den)

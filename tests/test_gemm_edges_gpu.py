@@ -64,7 +64,8 @@ def test_narrow_operands(ctx, M, N, K, ta, tb, pad):
 
 
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
-@pytest.mark.parametrize("M,N,K", [(33, 17000, 67), (17000, 61, 97), (16500, 17, 19)])
+@pytest.mark.parametrize("M,N,K", [(33, 17000, 67), (17000, 61, 97), (16500, 17, 19),
+                                   (16450, 70, 40)])  # (column sums of over 256 partial rows)
 def test_narrow_epilogues(ctx, M, N, K, ta, tb):
     test_epilogues(ctx, M, N, K, ta, tb)
 
