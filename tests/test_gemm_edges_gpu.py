@@ -1,6 +1,7 @@
 """GEMMs of odd extents and leading dimensions on every kernel and plan that takes them: the
-direct-to-LDS kernel's unaligned form (tiles moved back at the operand's end, the chunk K cuts),
-the register kernel's 32x32 and 64x64 tiles with their K groups, and split-K slices of both.
+direct-to-LDS kernel's unaligned form (tiles moved back at the operand's end, the chunk K cuts,
+operands of less than a tile), the register kernel's 32x32 and 64x64 tiles with their K groups, and
+split-K slices of both.
 Operands are small integers, so every product sum is exact and the results must be equal bit for
 bit, whatever the order of the sums; each epilogue is checked the same way."""
 import numpy as np
@@ -15,7 +16,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [
     (17, 17, 17), (33, 47, 31), (100, 101, 129),   # 32x32 tiles, K below and above a step a wave
     (97, 301, 515), (20, 21, 2001),                # ... in slices
-    (1023, 1025, 19),                              # 64x64 register tiles or LDS tiles by layout
+    (1023, 1025, 19),                              # 64x64 LDS tiles, one k-tile
     (1025, 513, 67), (575, 1087, 33), (512, 1024, 1027),  # 64x64 LDS tiles, whole and in slices
     (2047, 2047, 35), (2049, 2050, 34),            # 128x128 LDS tiles; 64x64 past their last round
     (385, 387, 2051), (65, 130, 1100),             # deep: slices of 64x64 tiles
