@@ -424,8 +424,8 @@ __global__ void __launch_bounds__(256) colsum_fold(double* part, int64_t P, int6
     part[r0 * N + col] = ((lds[0][lane] + lds[1][lane]) + lds[2][lane]) + lds[3][lane];
 }
 // Column sums, pass 2: block x finishes 64 columns of P partial rows `step` apart; wave w adds
-// partial rows w, w + 4, ... in two interleaved chains (independent loads in flight), then the chains and the four waves are
-// combined in a fixed order, so results are run-to-run identical.
+// partial rows w, w + 4, ... in two interleaved chains (independent loads in flight), then the
+// chains and the four waves are combined in a fixed order, so results are run-to-run identical.
 __global__ void __launch_bounds__(256) colsum_pass2(const double* part, float* out, int64_t P,
                                                     int64_t N, int64_t step, double divisor,
                                                     int accumulate) {
@@ -879,7 +879,8 @@ hipError_t launch_colsum(const float* x, float* out, int64_t R, int64_t N, int64
   if (P > 0) {
     if (N > CS_COLS) {  // (64 columns fill colsum_pass1's lanes: [1000000, 33] 120 us, 144 in fours)
       dim3 g1((unsigned)((N + 4 * CS_COLS - 1) / (4 * CS_COLS)), (unsigned)P);
-      if (R <= CS_FEW_ROWS)
+      // (sixteen waves of 2^30 and more columns are more threads than a grid dimension holds)
+      if (R <= CS_FEW_ROWS || N >= (1ll << 30) - 4 * CS_COLS)
         hipLaunchKernelGGL(colsum_pass1_v4<4>, g1, dim3(256), 0, s, x, partial, R, N, ldx, rows);
       else
         hipLaunchKernelGGL(colsum_pass1_v4<16>, g1, dim3(1024), 0, s, x, partial, R, N, ldx, rows);
