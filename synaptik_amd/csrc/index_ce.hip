@@ -11,7 +11,7 @@
 //
 // The gradient is scaled by the sample count, which is R without an ignore index. With one, up to
 // a stated number of rows each workgroup counts the targets itself; beyond that a launch before
-// counts them once.
+// counts them once. The mean counts the rows that it adds.
 //
 // Row statistics: the loss shifts by the maximum by '>' and the gradient by Math.max. A NaN
 // logit makes both NaN through the sum, and the sign of a zero maximum changes no exponential,
@@ -28,7 +28,7 @@ struct CeArgs {
   const float* logits;
   const void* target;
   float* grad;      // null: the loss alone
-  float* row_loss;  // [R]: lse - logit of the target, 0 where ignored or out of bounds
+  float* row_loss;  // [R]: lse - logit of the target, CE_NO_LOSS where ignored or out of bounds
   const uint4* count;  // sample counts of four parts of the rows; null: counted here (with an
                        // ignore index) or R
   uint32_t* status;
@@ -36,6 +36,11 @@ struct CeArgs {
   int has_ignore;
   float g;
 };
+
+// The loss of a row that is not a sample: -0, which the sum does not see and no sample's loss is (a
+// difference is -0 only for -0 minus +0, and lse = m + log(sum), log(sum) >= +0, is never -0).
+constexpr float CE_NO_LOSS = -0.0f;
+__device__ __forceinline__ int ce_no_loss(float v) { return __float_as_uint(v) == 0x80000000u; }
 
 template <typename T, int NT>
 __device__ __forceinline__ double ce_count(const CeArgs& a, int64_t first, int64_t end, double* dl) {
@@ -80,7 +85,7 @@ __global__ void __launch_bounds__(256) ce_rows_wave(CeArgs a) {
   const bool ignored = a.has_ignore && t == a.ignore;
   const bool in_range = t >= 0 && t < a.C;
   if (ignored) {  // (uniform for the wave) no loss, a zero gradient: the row is not read
-    if (lane == 0) a.row_loss[r] = 0.0f;
+    if (lane == 0) a.row_loss[r] = CE_NO_LOSS;
     if (a.grad != nullptr) {
 #pragma unroll
       for (int i = 0; i < V; ++i)
@@ -112,7 +117,7 @@ __global__ void __launch_bounds__(256) ce_rows_wave(CeArgs a) {
   if (lane == 0) {
     if (!in_range) atomicOr(a.status, (uint32_t)DEV_INDEX_OUT_OF_BOUNDS);
     const float lse = m + (float)log((double)sum);
-    a.row_loss[r] = in_range ? lse - xt : 0.0f;
+    a.row_loss[r] = in_range ? lse - xt : CE_NO_LOSS;
   }
   if (a.grad == nullptr) return;
   float* gr = a.grad + r * a.C;
@@ -142,7 +147,7 @@ ce_rows_block(CeArgs a) {
     const int safe = (int)(t < 0 ? 0 : (t >= a.C ? a.C - 1 : t));
     const RowGroups view(row, C);
     if (ignored) {  // no loss, a zero gradient: the row is not read
-      if (threadIdx.x == 0) a.row_loss[r] = 0.0f;
+      if (threadIdx.x == 0) a.row_loss[r] = CE_NO_LOSS;
       if (a.grad != nullptr)
         for (int q = threadIdx.x; q < view.groups; q += NT)
           view.store(a.grad + r * a.C, q, make_float4(0.f, 0.f, 0.f, 0.f));
@@ -184,7 +189,7 @@ ce_rows_block(CeArgs a) {
     if (threadIdx.x == 0) {
       if (!in_range) atomicOr(a.status, (uint32_t)DEV_INDEX_OUT_OF_BOUNDS);
       const float lse = m + (float)log((double)sum);
-      a.row_loss[r] = in_range ? lse - xt : 0.0f;
+      a.row_loss[r] = in_range ? lse - xt : CE_NO_LOSS;
     }
     if (a.grad == nullptr) continue;
     const float inv = 1.0f / sum;
@@ -219,7 +224,7 @@ __global__ void __launch_bounds__(CE_STREAM_NT) ce_rows_stream(CeArgs a) {
     const bool ignored = a.has_ignore && t == a.ignore;
     const bool in_range = t >= 0 && t < a.C;
     if (ignored) {  // as in ce_rows_block
-      if (threadIdx.x == 0) a.row_loss[r] = 0.0f;
+      if (threadIdx.x == 0) a.row_loss[r] = CE_NO_LOSS;
       if (a.grad != nullptr)
         for (int64_t c = threadIdx.x; c < a.C; c += NT) a.grad[r * a.C + c] = 0.0f;
       continue;
@@ -242,7 +247,7 @@ __global__ void __launch_bounds__(CE_STREAM_NT) ce_rows_stream(CeArgs a) {
     if (threadIdx.x == 0) {
       if (!in_range) atomicOr(a.status, (uint32_t)DEV_INDEX_OUT_OF_BOUNDS);
       const float lse = m + (float)log((double)sum);
-      a.row_loss[r] = in_range ? lse - xt : 0.0f;
+      a.row_loss[r] = in_range ? lse - xt : CE_NO_LOSS;
     }
     if (a.grad == nullptr) continue;
     const float inv = 1.0f / sum;
@@ -264,32 +269,55 @@ __global__ void __launch_bounds__(1024) ce_count_kernel(CeArgs a, uint32_t* coun
 }
 
 // The MEAN: binary64 partials of rows 4i .. 4i+3 summed in a fixed order, one rounding, over the
-// sample count.
-template <typename T>
-__global__ void __launch_bounds__(256) ce_finish_kernel(CeArgs a, float* loss) {
-  __shared__ double dl[4];
-  const float divisor = ce_divisor<T, 256>(a, dl);
-  __syncthreads();
-  const int64_t P = (a.R + 3) / 4, whole = a.R / 4;
-  const float4* quad = reinterpret_cast<const float4*>(a.row_loss);  // (16-byte aligned)
+// number of samples, which with an ignore index is counted from the same losses. Bound by latency:
+// eight loads are in flight whatever the number of rows, those past the end reading the last group,
+// and up to CE_FINISH_ROWS_WAVE rows, which one wave holds, no other wave is waited for.
+// [5120, 140] with an ignore index, the loss alone: 15.6 us a step on MI355X when this block read the
+// targets to count them, 8.5 so.
+constexpr int64_t CE_FINISH_ROWS_WAVE = 252;
+template <int NT>
+__global__ void __launch_bounds__(NT) ce_finish_kernel(const float* __restrict__ row_loss, int64_t R,
+                                                       int has_ignore, float* loss) {
+  __shared__ double dl[NT / 64];
+  __shared__ int kl[NT / 64];
+  const int64_t whole = R / 4;
+  const float4* quad = reinterpret_cast<const float4*>(row_loss);  // (16-byte aligned)
   double s = 0.0;
-  int64_t i = threadIdx.x;
-  for (; i + 7 * 256 < whole; i += 8 * 256) {  // eight loads in flight, added in order
+  int skipped = 0;
+  for (int64_t i = threadIdx.x; i < whole; i += 8 * 256) {
     float4 v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = quad[i + u * 256];
+    for (int u = 0; u < 8; ++u) v[u] = quad[min(i + u * 256, whole - 1)];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      s += (((double)v[u].x + (double)v[u].y) + (double)v[u].z) + (double)v[u].w;
+    for (int u = 0; u < 8; ++u) {
+      if (i + u * 256 < whole) {
+        s += (((double)v[u].x + (double)v[u].y) + (double)v[u].z) + (double)v[u].w;
+        skipped += ce_no_loss(v[u].x) + ce_no_loss(v[u].y) + ce_no_loss(v[u].z) + ce_no_loss(v[u].w);
+      }
+    }
   }
-  for (; i < P; i += 256) {
+  if (R % 4 != 0 && (int)threadIdx.x == (int)(whole % 256)) {  // the thread whose turn it is
     double q[4];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) q[w] = 4 * i + w < a.R ? (double)a.row_loss[4 * i + w] : 0.0;
+    for (int w = 0; w < 4; ++w) {
+      const float v = 4 * whole + w < R ? row_loss[4 * whole + w] : 0.0f;
+      q[w] = (double)v;
+      skipped += ce_no_loss(v);
+    }
     s += ((q[0] + q[1]) + q[2]) + q[3];
   }
-  s = block_sum<256>(s, dl);
-  if (threadIdx.x == 0) loss[0] = (float)s / divisor;
+  s = wave_sum(s);
+  if (has_ignore) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) skipped += __shfl_xor(skipped, o, 64);
+  }
+  if constexpr (NT > 64) {
+    if ((threadIdx.x & 63) == 0) { dl[threadIdx.x >> 6] = s; kl[threadIdx.x >> 6] = skipped; }
+    __syncthreads();
+    s = ((dl[0] + dl[1]) + dl[2]) + dl[3];
+    skipped = (kl[0] + kl[1]) + (kl[2] + kl[3]);
+  }
+  if (threadIdx.x == 0) loss[0] = (float)s / (float)(double)(R - (has_ignore ? skipped : 0));
 }
 
 // Rows a workgroup counts by itself instead of a launch before: with one row a wave at most 1024
@@ -312,8 +340,8 @@ void launch_block(const CeArgs& a, hipStream_t s) {
 template <typename T>
 hipError_t launch_typed(CeArgs a, float* loss, uint32_t* count, hipStream_t s) {
   const bool wave = a.C <= CE_WAVE_CLASSES;
-  // (without a gradient only the last launch counts)
-  if (a.has_ignore && a.R > (wave || a.grad == nullptr ? CE_COUNT_ROWS_WAVE : CE_COUNT_ROWS_BLOCK)) {
+  // (only a gradient is scaled before the mean is formed)
+  if (a.has_ignore && a.grad != nullptr && a.R > (wave ? CE_COUNT_ROWS_WAVE : CE_COUNT_ROWS_BLOCK)) {
     hipLaunchKernelGGL(ce_count_kernel<T>, dim3(4), dim3(1024), 0, s, a, count);
     a.count = reinterpret_cast<const uint4*>(count);
   }
@@ -334,7 +362,10 @@ hipError_t launch_typed(CeArgs a, float* loss, uint32_t* count, hipStream_t s) {
   else
     hipLaunchKernelGGL(ce_rows_stream<T>, dim3((unsigned)std::min<int64_t>(a.R, 1 << 20)),
                        dim3(CE_STREAM_NT), 0, s, a);
-  hipLaunchKernelGGL(ce_finish_kernel<T>, dim3(1), dim3(256), 0, s, a, loss);
+  if (a.R <= CE_FINISH_ROWS_WAVE)
+    hipLaunchKernelGGL(ce_finish_kernel<64>, dim3(1), dim3(64), 0, s, a.row_loss, a.R, a.has_ignore, loss);
+  else
+    hipLaunchKernelGGL(ce_finish_kernel<256>, dim3(1), dim3(256), 0, s, a.row_loss, a.R, a.has_ignore, loss);
   return hipGetLastError();
 }
 

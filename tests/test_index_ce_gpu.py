@@ -57,6 +57,34 @@ def test_sample_count_of_many_rows(ctx, R, C):
                                rtol=1e-5, atol=1e-9)
 
 
+@pytest.mark.parametrize("R", [1, 3, 4, 251, 252, 253, 1023, 1025, 8191, 8193, 8199])
+def test_mean_counts_samples_without_a_loss(ctx, R):
+    """The mean's loads at the edges of its rounds; samples whose loss is exactly zero (of either sign
+    of zero logits) count, ignored rows do not."""
+    print(f"[index_ce] mean R={R}", flush=True)
+    rng = np.random.default_rng(R)
+    logits = rng.standard_normal((R, 2)).astype(np.float32)
+    y = rng.integers(0, 2, R)
+    kind = rng.integers(0, 4, R)
+    kind[0] = 0
+    logits[kind == 1] = [-0.0, -np.inf]
+    logits[kind == 2] = [0.0, -200.0]
+    y[(kind == 1) | (kind == 2)] = 0
+    y[kind == 3] = -5
+    pb = ProgramBuilder()
+    sx, sy = pb.input(R * 2), pb.input(R, "i32")
+    both, alone, grad = pb.output(1), pb.output(1), pb.output(R * 2)
+    pb.index_ce(sx, sy, both, R, 2, grad=grad, ignore_index=-5)
+    pb.index_ce(sx, sy, alone, R, 2, ignore_index=-5)
+    valid = kind != 3
+    x = logits.astype(np.float64)
+    with np.errstate(divide="ignore"):
+        rows = np.log(np.exp(x).sum(1)) - x[np.arange(R), np.maximum(y, 0)]
+    a, b, _ = run_program(ctx, pb, [logits, y.astype(np.int32)], [both, alone, grad])
+    want = rows[valid].sum() / valid.sum()
+    assert abs(a[0] - want) <= 1e-6 * abs(want) + 1e-12 and a[0] == b[0]
+
+
 def test_special_rows(ctx):
     """NaN and infinite logits and a row of nothing but -inf, on both row forms."""
     for C in (70, 1500):
