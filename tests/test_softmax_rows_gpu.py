@@ -87,6 +87,27 @@ def test_backward(ctx, C):
 NANS = [0x7fc00000, 0x7fc00001, 0x7fffffff, 0xffffffff, 0x7f800001]
 
 
+@pytest.mark.parametrize("R,C", [(600, 900), (524288, 1), (524289, 1), (174763, 3), (131072, 4),
+                                 (104858, 5), (7825, 67), (1025, 512), (525, 1001), (3, 300001)])
+def test_log_sum_exp_gradient(ctx, R, C):
+    """An element a thread below 2^19 elements or four columns, else groups of four over row ends."""
+    print(f"[lse bwd] {R}x{C}", flush=True)
+    rng = np.random.default_rng(R)
+    x = rng.standard_normal((R, C)).astype(np.float32)
+    lse, g = rng.standard_normal(R).astype(np.float32), rng.standard_normal(R).astype(np.float32)
+    x[0, 0], x[R // 2, C - 1], x[R - 1, C - 1] = np.nan, np.inf, -np.inf
+    pb = ProgramBuilder()
+    sx, sl, sg = pb.input(R * C), pb.input(R), pb.input(R)
+    each, same = pb.output(R * C), pb.output(R * C)
+    pb.lse_bwd(sx, sl, each, R, C, g=sg)
+    pb.lse_bwd(sx, sl, same, R, C, gconst=0.75)
+    a, b = run_program(ctx, pb, [x, lse, g], [each, same])
+    e = np.exp((x - lse[:, None]).astype(np.float64))
+    # the exponential's rounding (up to one unit) and the product's
+    np.testing.assert_allclose(a.reshape(R, C), g[:, None] * e, rtol=2e-7)
+    np.testing.assert_allclose(b.reshape(R, C), 0.75 * e, rtol=2e-7)
+
+
 @pytest.mark.parametrize("log", [False, True])
 @pytest.mark.parametrize("C", [2, 101, 252, 512, 1021, 2044, 4096, 5003, 20001, 32768, 40000])
 def test_every_nan_pattern_takes_its_row(ctx, C, log):
