@@ -633,6 +633,27 @@ __global__ void __launch_bounds__(256) lse_bwd_kernel(const float* __restrict__ 
     dx[i] = gr * exp_rn(x[i] - lse[r]);
   }
 }
+__global__ void __launch_bounds__(256) lse_bwd_groups(const float* __restrict__ x,
+                                                      const float* __restrict__ lse, const float* g,
+                                                      float gconst, float* __restrict__ dx, int64_t R,
+                                                      int64_t C) {
+  const int64_t n = R * C;
+  for (int64_t i = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x); i < n;
+       i += 4 * (int64_t)gridDim.x * blockDim.x) {
+    const int64_t r = n <= 0xffffffffll ? (int64_t)((uint32_t)i / (uint32_t)C) : i / C;
+    const int64_t next = min<int64_t>(r + 1, R - 1), left = C - (i - r * C);  // left: in row r
+    const float l0 = lse[r], l1 = lse[next];
+    const float g0 = g != nullptr ? g[r] : gconst, g1 = g != nullptr ? g[next] : gconst;
+    auto element = [&](float v, int q) { return (q < left ? g0 : g1) * exp_rn(v - (q < left ? l0 : l1)); };
+    if (i + 3 < n) {
+      const float4u v = __builtin_nontemporal_load(reinterpret_cast<const float4u*>(x + i));
+      const float4u o = {element(v[0], 0), element(v[1], 1), element(v[2], 2), element(v[3], 3)};
+      __builtin_nontemporal_store(o, reinterpret_cast<float4u*>(dx + i));
+    } else {
+      for (int q = 0; i + q < n; ++q) dx[i + q] = element(x[i + q], q);
+    }
+  }
+}
 
 // ---- MSE (CpuLossReferenceKernel.java:67-87, LossGradientRules.java:77-97) ----
 constexpr int MSE_BLOCKS = 1024;
@@ -721,6 +742,15 @@ void launch_bwd_rows(const float* y, const float* g, float* dx, int64_t R, int64
 }
 // Floats that V groups of each of NT threads hold, whatever the row's start.
 constexpr int64_t row_capacity(int nt, int v) { return 4ll * nt * v - 4; }
+// Backward, rows of at most 2044: up to this many rows a workgroup of 256 a row ends sooner than a
+// wave a row, which holds ragged groups: the streamed form or, for aligned rows, the one in
+// registers. us a step on MI355X, streamed and a wave a row: [16, 275] 3.2 and 4.3, [2048, 275] 4.6
+// and 4.8, [2048, 907] 6.4 and 7.2, [512, 130] 3.2 and 3.4, [1024, 1691] 6.5 and 6.9; [4096, 275]
+// 6.3 and 5.3, [1544, 130] 3.8 and 3.7, [1544, 1691] 8.6 and 8.5. Aligned rows of at most 252 take a
+// wave each from the first ([16, 200] 3.1 and 2.9).
+inline int64_t sb_few_rows(int64_t C) {
+  return C > row_capacity(64, 1) && C <= row_capacity(64, 4) ? 2048 : 1024;
+}
 }  // namespace
 
 hipError_t launch_softmax_fwd(const float* x, float* y, float* lse, int64_t R, int64_t C,
@@ -767,7 +797,11 @@ hipError_t launch_softmax_bwd(const float* y, const float* g, float* dx, int64_t
   };
   using std::integral_constant;
   if (C <= 0) return hipSuccess;
-  if (C <= row_capacity(64, 1)) rows(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+  if ((!vec && C <= row_capacity(64, 8) && R <= sb_few_rows(C)) || C > row_capacity(1024, 8) + (vec ? 4 : 0))
+    hipLaunchKernelGGL(softmax_bwd_stream, dim3((unsigned)R), dim3(SM_NT), 0, s, y, g, dx, C, rowscale,
+                       rowscale_const);
+  else if (C <= row_capacity(64, 1)) rows(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+  else if (vec && C <= 508 && R <= 1024) regs(integral_constant<int, 1>{});
   else if (C <= row_capacity(64, 2)) rows(integral_constant<int, 64>{}, integral_constant<int, 2>{});
   else if (vec && C <= 1024) regs(integral_constant<int, 1>{});
   else if (vec && C <= 2048) regs(integral_constant<int, 2>{});
@@ -785,8 +819,10 @@ hipError_t launch_lse_bwd(const float* x, const float* lse, const float* g, floa
                           float* dx, int64_t R, int64_t C, hipStream_t s) {
   const int64_t n = R * C;
   if (n <= 0) return hipSuccess;
-  const unsigned blocks = (unsigned)std::min<int64_t>(65536, (n + 255) / 256);
-  hipLaunchKernelGGL(lse_bwd_kernel, dim3(blocks), dim3(256), 0, s, x, lse, g, gconst, dx, R, C);
+  const int each = n >= LSE_BWD_GROUPED && C >= 4 ? 4 : 1;
+  const dim3 blocks((unsigned)std::min<int64_t>(65536, (n + 256 * each - 1) / (256 * each))), nt(256);
+  if (each == 4) hipLaunchKernelGGL(lse_bwd_groups, blocks, nt, 0, s, x, lse, g, gconst, dx, R, C);
+  else hipLaunchKernelGGL(lse_bwd_kernel, blocks, nt, 0, s, x, lse, g, gconst, dx, R, C);
   return hipGetLastError();
 }
 

@@ -62,9 +62,8 @@ def test_forward(ctx, C, log):
 
 
 @pytest.mark.parametrize("C", WIDTHS)
-def test_backward(ctx, C):
-    print(f"[softmax bwd] C={C}", flush=True)
-    R = 6
+def test_backward(ctx, C, R=6):
+    print(f"[softmax bwd] C={C} R={R}", flush=True)
     rng = np.random.default_rng(C + 1)
     y = oracle.softmax_rows((rng.standard_normal((R, C)) * 2).astype(np.float32))
     g = rng.standard_normal((R, C)).astype(np.float32)
@@ -85,6 +84,13 @@ def test_backward(ctx, C):
 # NaN bit patterns: numpy's, the ones whose low payload bits are set, and memory poison. A row is in
 # the binary32 exponential's range but for its NaN.
 NANS = [0x7fc00000, 0x7fc00001, 0x7fffffff, 0xffffffff, 0x7f800001]
+
+
+@pytest.mark.parametrize("R", [1024, 1025, 2048, 2049])
+@pytest.mark.parametrize("C", [1, 5, 200, 253, 400, 509, 1020, 1021, 2043])
+def test_backward_of_many_rows(ctx, C, R):
+    """Rows of at most 2044: a workgroup a row up to 1024 or 2048 rows, a wave a row beyond."""
+    test_backward(ctx, C, R)
 
 
 @pytest.mark.parametrize("R,C", [(600, 900), (524288, 1), (524289, 1), (174763, 3), (131072, 4),
