@@ -327,6 +327,11 @@ __global__ void __launch_bounds__(256) colsum_pass1(const float* __restrict__ x,
 // [20000, 1001] 40.8 us on MI355X, 21.7 so. Up to CS_FEW_ROWS rows four waves do: the others
 // would only be launched and waited for ([8, 1000000] 27.3 us a call against 33.4).
 constexpr int64_t CS_FEW_ROWS = 32;
+// Few unaligned rows go to colsum_pass1, whose four times as many blocks are done sooner than a
+// lane's four ragged columns. us a step, there and here: [16, 301] 4.5 and 5.0, [32, 1001] 4.8 and
+// 5.7, [33, 100001] 6.0 and 6.5, [2, 1000001] 12.1 and 14.0; [64, 301] 5.7 and 5.4, [16, 1000001]
+// 24.6 and 22.2.
+constexpr int64_t CS_FEW_UNALIGNED = 48, CS_FEW_COLS = 1 << 18;
 template <int CS_WAVES>
 __global__ void __launch_bounds__(64 * CS_WAVES) colsum_pass1_v4(const float* __restrict__ x,
                                                                 double* part, int64_t R, int64_t N,
@@ -877,7 +882,9 @@ hipError_t launch_colsum(const float* x, float* out, int64_t R, int64_t N, int64
   const int64_t rows = colsum_rows_per_panel(R, N);
   const int64_t P = (R + rows - 1) / rows;
   if (P > 0) {
-    if (N > CS_COLS) {  // (64 columns fill colsum_pass1's lanes: [1000000, 33] 120 us, 144 in fours)
+    const bool aligned = N % 4 == 0 && ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0;
+    // (64 columns fill colsum_pass1's lanes: [1000000, 33] 120 us, 144 in fours)
+    if (N > CS_COLS && (aligned || R > CS_FEW_UNALIGNED || (R > 4 && N > CS_FEW_COLS))) {
       dim3 g1((unsigned)((N + 4 * CS_COLS - 1) / (4 * CS_COLS)), (unsigned)P);
       // (sixteen waves of 2^30 and more columns are more threads than a grid dimension holds)
       if (R <= CS_FEW_ROWS || N >= (1ll << 30) - 4 * CS_COLS)

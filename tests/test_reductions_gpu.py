@@ -45,9 +45,11 @@ def test_row_reductions(ctx, C):
 
 
 @pytest.mark.parametrize("R,N", [(40000, 64), (40000, 65), (40001, 100), (33000, 255), (32, 300),
-                                 (33, 300), (1, 1000)])
+                                 (33, 300), (1, 1000), (32, 301), (48, 301), (49, 301), (2, 262143),
+                                 (48, 262145), (4, 262145), (5, 262145)])
 def test_column_sums_at_the_dispatch_edges(ctx, R, N):
-    """4-byte lanes up to 64 columns, four columns a lane beyond; four waves up to 32 rows."""
+    """4-byte lanes up to 64 columns, for up to 48 unaligned rows of at most 2^18 columns and for up to
+    four of any width; four columns a lane beyond, on four waves up to 32 rows."""
     test_column_sums(ctx, R, N, 0)
 
 
