@@ -816,11 +816,15 @@ inline int v2_choose(const GemmParams& p, bool aligned) {
 
 // In-workgroup split-K (KS = 2): fewer than two workgroups per CU and at least eight k-tiles per
 // group. Eight waves give each SIMD two, as two four-wave workgroups per CU would, without more
-// partials in HBM. 128x128 tiles only on split-K slices.
-inline bool v2_split_in_group(const GemmParams& p, int bt, int64_t tiles, int64_t slices) {
+// partials in HBM. 128x128 tiles only on split-K slices. Operands of less than a tile (cut) from four
+// k-tiles per group, with a staged update, which the groups share, from three: one wave a SIMD was
+// slower there than the register kernel before (us a step on MI355X, one group and two: 16968x31x509
+// TN 34.8 and 28.6, with an SGD update 40.3 and 32.2; 20001x63x313 TN 24.4 and 20.5; 20001x27x200 TN
+// with an update 24.6 and 21.8, without 18.5 and 18.6, 16968x27x200 16.8 and 17.6).
+inline bool v2_split_in_group(const GemmParams& p, int bt, int64_t tiles, int64_t slices, bool cut) {
   const int64_t span = p.kchunk > 0 ? p.kchunk : p.K;
   return v2_ks2_enabled() && (bt == 64 || (p.kchunk > 0 && p.partial != nullptr)) &&
-         tiles * slices < 512 && span >= 16 * V2_BK;
+         tiles * slices < 512 && span >= (!cut ? 16 : p.upd.pn != nullptr ? 6 : 8) * V2_BK;
 }
 
 template <bool TA, bool TB, int BT, bool U>
@@ -828,11 +832,12 @@ hipError_t launch_v2_bt(const GemmParams& p, hipStream_t s) {
   const unsigned tiles = (unsigned)(((p.M + BT - 1) / BT) * ((p.N + BT - 1) / BT));
   const unsigned slices = p.kchunk > 0 ? (unsigned)((p.K + p.kchunk - 1) / p.kchunk) : 1u;
   const int64_t span = p.kchunk > 0 ? p.kchunk : p.K;
-  const bool ks2 = !(U && BT == 128) && v2_split_in_group(p, BT, tiles, slices);
+  const bool cut = U && BT == 64 && ((TA && p.M < BT) || (!TB && p.N < BT));
+  const bool ks2 = !(U && BT == 128) && v2_split_in_group(p, BT, tiles, slices, cut);
   g_colsum_rows = ((p.M + BT - 1) / BT) * (ks2 ? 4 : 2);  // per wave row and K group
   const dim3 grid(tiles, slices), block(ks2 ? 2 * V2_NT : V2_NT);
   if constexpr (U && BT == 64 && (TA || !TB)) {
-    if ((TA && p.M < BT) || (!TB && p.N < BT)) {
+    if (cut) {
       if (ks2)
         hipLaunchKernelGGL((gemm_f32_v2<!TA, TB, 64, true, 2, true, true>), grid, block, 0, s, p);
       else

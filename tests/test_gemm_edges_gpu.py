@@ -54,6 +54,7 @@ def test_exact_products(ctx, M, N, K, ta, tb, pad):
 # M/N-contiguous operands of less than a 64-wide tile, many tiles along the other extent: LDS tiles
 # whose chunks run past the operand's row, 64x64 register tiles (the last three), by layout and K
 NARROW = [(33, 17000, 67), (17000, 63, 97), (61, 16500, 520), (20, 16500, 200), (33000, 33, 33),
+          (27, 16500, 313), (16500, 45, 257),            # ... in two K groups a workgroup
           (16500, 17, 19), (31, 16500, 19), (16385, 32, 127)]
 
 
@@ -66,6 +67,7 @@ def test_narrow_operands(ctx, M, N, K, ta, tb, pad):
 
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
 @pytest.mark.parametrize("M,N,K", [(33, 17000, 67), (17000, 61, 97), (16500, 17, 19),
+                                   (16450, 27, 200), (27, 16450, 313), (16450, 45, 257),
                                    (16450, 70, 40)])  # (column sums of over 256 partial rows)
 def test_narrow_epilogues(ctx, M, N, K, ta, tb):
     test_epilogues(ctx, M, N, K, ta, tb)
